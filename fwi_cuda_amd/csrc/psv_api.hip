@@ -144,6 +144,17 @@ struct fwi_ctx {
     int depth = 1; // rows the one-pass step loads ahead (autotuned)
     std::string tune_log;
 
+    // ---- the resident propagation (psv_resident.h): tilings per batch size, FP32 and FP64
+    // (shots 0: none), edge words, the next launch's first tag, flag of a wait that gave up
+    bool res_grid = false;   // the grid, acquisition and device allow it
+    int cus = 0;
+    std::vector<int> zmap_h, xmap_h;
+    std::map<int, ResPlan> rplan, rplan64;
+    unsigned long long *mail = nullptr;
+    size_t mail_words = 0;
+    uint32_t mail_tag = 1;
+    int *res_err = nullptr;  // pinned host memory
+
     // ---- profiling
     int prof_on = 0, prof_stride = 1;
     std::vector<hipEvent_t> ev_pool;
@@ -257,6 +268,10 @@ int sync(fwi_ctx *c) {
     e = hipGetLastError();
     if (e != hipSuccess) return c->fail(FWI_EHIP, "launch: %s", hipGetErrorString(e));
     prof_collect(c);
+    if (c->res_err && *(volatile int *)c->res_err) {
+        *c->res_err = 0;
+        return c->fail(FWI_EHIP, "resident propagation: a tile's neighbour did not answer");
+    }
     return FWI_OK;
 }
 
@@ -415,6 +430,125 @@ RecArgs rec_args(fwi_ctx *c, int s0, int nb) {
     return r;
 }
 
+// ---------------------------------------------------------------------------
+// the resident propagation
+// ---------------------------------------------------------------------------
+constexpr int kFlushSteps = 64;   // adjoint steps between flushes of the FP32 correlation sums
+
+// The tiling of the resident propagation for a batch of nb shots, or null where it does not
+// apply: a pinned kernel variant, rows or work order; a surface other than the top one at
+// row N, or a source or receiver outside the interior (the one-pass step's conditions); a
+// grid whose shot does not fit the chip's LDS.  Whether it applies does not depend on nb,
+// storage, graph replay or profiling: every pass of a context takes the same kernels.
+const ResPlan *resident_plan(fwi_ctx *c, int nb, bool fp64) {
+    if (!c->res_grid || c->plain || (!fp64 && (c->o.kernel_variant || c->o.tile_tz > 0 || c->o.work_order))) return nullptr;
+    auto &cache = fp64 ? c->rplan64 : c->rplan;
+    auto it = cache.find(nb);
+    if (it == cache.end()) {
+        ResPlan p{};
+        if (!plan_resident(c->g.nz, c->g.nx, c->N, nb, fp64 ? 8 : 4, c->cus, kResLds, c->zmap_h, c->xmap_h, &p)) p.shots = 0;
+        it = cache.emplace(nb, p).first;
+    }
+    return it->second.shots > 0 ? &it->second : nullptr;
+}
+bool resident(fwi_ctx *c, int nb) { return resident_plan(c, nb, false) != nullptr; }
+
+// edge words for a tiling, and the first of n tags for a launch
+int resident_mail(fwi_ctx *c, const ResPlan &p, int elt, int n, uint32_t *tag) {
+    const size_t words = resident_words(p, c->N, elt);
+    if (words > c->mail_words) {
+        unsigned long long *m = c->dalloc<unsigned long long>(words);
+        if (!m) return c->fail(FWI_ENOMEM, "edge words of the resident propagation");
+        c->mail = m;
+        c->mail_words = words;
+        c->mail_tag = 0xffffffffu;   // cleared below
+    }
+    if (c->mail_tag > 0xffffffffu - (uint32_t)n - 1u) {
+        HIPCHK(hipMemsetAsync(c->mail, 0, c->mail_words * 8, c->st));
+        c->mail_tag = 1;
+    }
+    *tag = c->mail_tag;
+    c->mail_tag += (uint32_t)n + 1u;
+    return FWI_OK;
+}
+
+template <class T>
+void resident_grid_args(const fwi_ctx *c, ResArgs<T> &r, const ResPlan &p, int s0) {
+    r.nz = c->g.nz; r.nx = c->g.nx; r.P = c->P; r.nzs = c->nzs; r.nxs = c->nxs;
+    r.fs = c->fs();
+    r.shot0 = s0;
+    r.TX = p.TX; r.TZ = p.TZ; r.ntx = p.ntx; r.ntz = p.ntz;
+    r.psi_lds = p.psi_lds; r.psi_rows = p.psi_rows; r.psi_cols = p.psi_cols;
+    r.nt = c->g.nt;
+    r.dt = (T)c->g.dt;
+    for (int k = 0; k < 6; ++k) {
+        r.cz[k] = k < c->N ? (T)(c->g.hc[k + 1] / c->g.dz) : T(0);
+        r.cx[k] = k < c->N ? (T)(c->g.hc[k + 1] / c->g.dx) : T(0);
+    }
+    r.zp = c->zp;
+    r.xp = c->xp;
+    r.surf = c->surf_top_only ? c->N : -1;
+    r.snap_z1 = c->g.snap_z1; r.snap_z2 = c->g.snap_z2; r.snap_x1 = c->g.snap_x1; r.snap_x2 = c->g.snap_x2;
+    r.snap_dz = c->g.snap_dz; r.snap_dx = c->g.snap_dx; r.snap_dt = c->g.snap_dt;
+    r.snz = c->snz; r.snx = c->snx;
+    r.mail = c->mail;
+    r.err = c->res_err;
+}
+
+// Time indices t0, t0 + dir, ... (nsteps of them) of shots [s0, s0 + nb) on state w.
+// Forward (dir 1): snapshots into the slabs from time index tb on with store, velocity
+// samples into the rows of syn_* with record.  Adjoint (dir -1): correlation with the
+// slabs from tb on, flushed into the FP64 totals as flush_after says.
+int resident_steps(fwi_ctx *c, int s0, int nb, const Wave &w, int t0, int nsteps, int dir, float *We, bool store,
+                   int tb, bool record) {
+    if (nsteps <= 0) return FWI_OK;
+    const ResPlan &p = *resident_plan(c, nb, false);
+    const bool adj = dir < 0;
+    ResArgs<float> r{};
+    for (int a = 0; a < nb; a += p.shots) {
+        const int ns = std::min(p.shots, nb - a);
+        RETIF(resident_mail(c, p, 4, nsteps, &r.epoch));
+        resident_grid_args(c, r, p, s0);
+        r.s0 = a;
+        r.t0 = t0; r.nsteps = nsteps; r.dir = dir;
+        r.load = 1;
+        r.vz = w.f[0]; r.vx = w.f[1]; r.szz = w.f[2]; r.szx = w.f[3]; r.sxx = w.f[4];
+        r.uz = c->f[5]; r.ux = c->f[6]; r.We = We;
+        r.energy = We != nullptr;
+        for (int j = 0; j < 8; ++j) r.psi[j] = w.psi[j];
+        r.lam = c->lam; r.mu = c->mu; r.muzx = c->muzx; r.rhoz = c->rhoz; r.rhox = c->rhox;
+        r.store = store;
+        r.tb = tb;
+        for (int j = 0; j < 5; ++j) r.st[j] = c->snap[j], r.sn[j] = c->snap[j];
+        r.st_stride = r.sn_stride = c->snap_stride;
+        const size_t cells = (size_t)c->B * c->snz * c->snx;
+        float *g[5] = {c->gr[0], c->gr[1], c->gr[2], c->gx, c->gx + cells};
+        for (int j = 0; j < 5; ++j) r.g[j] = g[j];
+        r.g64 = c->gr64;
+        r.g64_stride = cells;
+        r.gform = c->gform;
+        r.flush_every = kFlushSteps;
+        r.gw = (float)(c->o.grad_sign * (double)c->g.snap_dt * c->g.dt);
+        r.gain_lm = (float)kGainLM;
+        r.src = adj ? adj_args(c, s0 + a, ns) : src_args(c, s0 + a, ns);
+        r.rec = adj_args(c, s0 + a, ns);
+        if (!record) r.rec.ngroups = 0;
+        r.seis_z = c->syn_z;
+        r.seis_x = c->syn_x;
+        Timer t(c, FWI_K_STEP);
+        HIPCHK(adj ? launch_resident_adjoint(r, p, c->N, ns, c->st) : launch_resident_forward(r, p, c->N, ns, c->st));
+    }
+    return FWI_OK;
+}
+
+// urec2's running sums of shots [s0, s0 + nb) from the velocity samples in syn_*
+void resident_seismograms(fwi_ctx *c, int s0, int nb) {
+    const int r0 = c->rec_off[s0], rows = c->rec_off[s0 + nb] - r0;
+    const size_t off = (size_t)r0 * c->g.nt;
+    Timer t(c, FWI_K_RECEIVER);
+    launch_seis_scan(c->syn_z + off, c->syn_x + off, rows, c->g.nt, c->g.dt, c->g.dz * c->g.dx, c->st);
+}
+
 // variants that advance a whole time step in one pass over two time levels
 bool one_pass(int var) { return var == 4 || var == 7 || var == 8 || var == 9; }
 
@@ -558,7 +692,7 @@ int zero_state(fwi_ctx *c, int nb, const Wave &w, bool u_we) {
     for (int i = 0; i < 5; ++i) HIPCHK(hipMemsetAsync(w.f[i], 0, sizeof(float) * nb * c->fs(), c->st));
     for (int i = 0; i < 4; ++i) HIPCHK(hipMemsetAsync(w.psi[i], 0, sizeof(float) * nb * c->psiz(), c->st));
     for (int i = 4; i < 8; ++i) HIPCHK(hipMemsetAsync(w.psi[i], 0, sizeof(float) * nb * c->psix(), c->st));
-    if (c->fusable) {   // the one-pass step never writes cells outside the interior: keep them zero
+    if (c->fusable && !resident(c, nb)) {   // the one-pass step never writes cells outside the interior: keep them zero
         for (int i = 0; i < 5; ++i) HIPCHK(hipMemsetAsync(w.f2[i], 0, sizeof(float) * nb * c->fs(), c->st));
         for (int i = 0; i < 2; ++i) HIPCHK(hipMemsetAsync(w.psi2[i], 0, sizeof(float) * nb * c->psiz(), c->st));
         for (int i = 2; i < 4; ++i) HIPCHK(hipMemsetAsync(w.psi2[i], 0, sizeof(float) * nb * c->psix(), c->st));
@@ -625,7 +759,7 @@ void take(fwi_ctx *c, const TuneVal &v) {
 }
 
 int autotune(fwi_ctx *c, int nb) {
-    if (c->plain || c->tuned) return FWI_OK;
+    if (c->plain || c->tuned || resident(c, nb)) return FWI_OK;
     const TuneKey key{c->g.nz, c->g.nx, c->N, nb};
     const int fv = c->o.kernel_variant;   // 0 = any
     const bool order_forced = c->o.work_order >= 1 && c->o.work_order <= 4;
@@ -772,12 +906,22 @@ int run_forward(fwi_ctx *c, int s0, int nb, bool store, bool record, bool energy
     // snapshots go to slab (it - tb) / snap_dt: every step with full storage, from t_keep
     // (a unit boundary) on with checkpoints
     const int tb = ckpt ? c->t_keep : 0;
+    const bool res = resident(c, nb);
     for (int it = 0; it < nt;) {
         if (ckpt && it % c->S == 0 && c->spine_slot[it / c->S] >= 0) {
             Timer t(c, FWI_K_STORE);
             RETIF(ckpt_copy(c, c->spine_slot[it / c->S], nb, w, true));
         }
         const bool keep = store && it >= tb;
+        if (res) {   // to the next state to save, or the end
+            int t1 = nt;
+            if (ckpt)
+                for (t1 = std::min(nt, (it / c->S + 1) * c->S); t1 < nt && c->spine_slot[t1 / c->S] < 0;)
+                    t1 = std::min(nt, t1 + c->S);
+            RETIF(resident_steps(c, s0, nb, w, it, t1 - it, 1, energy ? c->f[7] : nullptr, store, tb, record));
+            it = t1;
+            continue;
+        }
         if (graph && it + K <= nt) {
             KArgs ag = a;
             ag.si = c->si_fwd;
@@ -803,6 +947,7 @@ int run_forward(fwi_ctx *c, int s0, int nb, bool store, bool record, bool energy
         }
         ++it;
     }
+    if (res && record) resident_seismograms(c, s0, nb);
     c->last_s0 = s0;
     c->last_nb = nb;
     return check_finite(c, nb);
@@ -843,7 +988,6 @@ void adj_step(fwi_ctx *c, KArgs &a, const Wave &w, const SrcArgs &sa, int it, si
 // The FP32 correlation sums go into their FP64 totals after the adjoint step of every time
 // index t with (nt - t) % kFlushSteps == 0 and once at the end: the same time steps whatever
 // the storage, so full storage, checkpoints and graph replay group the FP32 partial sums alike.
-constexpr int kFlushSteps = 64;
 static_assert(kGraphChunk == kFlushSteps, "a full-storage graph chunk ends on a flush step");
 
 bool flush_after(int nt, int it) { return (nt - it) % kFlushSteps == 0; }
@@ -888,7 +1032,11 @@ int run_adjoint(fwi_ctx *c, int s0, int nb) {
     ag.si_base = c->si_base;
     ag.si_dir = -1;
     ChunkGraph cga(c);
-    if (c->storage != FWI_STORE_CHECKPOINT) {
+    const bool res = resident(c, nb);
+    if (c->storage != FWI_STORE_CHECKPOINT && res) {
+        RETIF(resident_steps(c, s0, nb, w, nt - 1, nt, -1, c->f[8], false, 0, false));
+        if (nt % kFlushSteps) flush_sums(c, nb);
+    } else if (c->storage != FWI_STORE_CHECKPOINT) {
         const int K = kGraphChunk;
         const bool graph = use_graphs(c);
         for (int jt = 0; jt < nt;) {
@@ -937,6 +1085,7 @@ int run_adjoint(fwi_ctx *c, int s0, int nb) {
         };
         // units [u0, u0 + k) forward from the state in rw, nothing stored (never the last unit)
         auto advance = [&](int u0, int k) -> int {
+            if (res) return resident_steps(c, s0, nb, rw, u0 * S, k * S, 1, nullptr, false, 0, false);
             for (int u = u0; u < u0 + k; ++u) {
                 const int t0 = u * S;
                 if (graph) {
@@ -955,6 +1104,7 @@ int run_adjoint(fwi_ctx *c, int s0, int nb) {
         // the adjoint steps of unit u, its snapshots in the buffer from time step tb on
         auto adjoint_unit = [&](int u, int tb) -> int {
             const int t0 = u * S, t1 = std::min(t0 + S, nt);
+            if (res) return resident_steps(c, s0, nb, w, t1 - 1, t1 - t0, -1, c->f[8], false, tb, false);
             if (graph && t1 - t0 == S) {   // the step table places the slabs
                 return cga.run(t1 - 1, [&]() {
                     for (int j = 0; j < S; ++j) {
@@ -973,6 +1123,10 @@ int run_adjoint(fwi_ctx *c, int s0, int nb) {
         // unit u recomputed from the state in rw into the segment buffer, then its adjoint steps
         auto leaf = [&](int u) -> int {
             const int t0 = u * S, t1 = std::min(t0 + S, nt);
+            if (res) {
+                RETIF(resident_steps(c, s0, nb, rw, t0, t1 - t0, 1, nullptr, true, t0, false));
+                return adjoint_unit(u, t0);
+            }
             if (graph && t1 - t0 == S) {
                 RETIF(cgr.run(t0, [&]() {
                     for (int j = 0; j < S; ++j) {
@@ -1094,6 +1248,29 @@ int run_forward64(fwi_ctx *c, int s0, int nb) {
     HIPCHK(hipMemsetAsync(c->acc, 0, sizeof(double) * 2 * c->nrec_tot, c->st));
     const SrcArgs sa = src_args(c, s0, nb);
     const RecArgs ra = rec_args(c, s0, nb);
+    if (const ResPlan *p = resident_plan(c, nb, true)) {
+        ResArgs<double> r{};
+        for (int a = 0; a < nb; a += p->shots) {
+            const int ns = std::min(p->shots, nb - a);
+            RETIF(resident_mail(c, *p, 8, nt, &r.epoch));
+            resident_grid_args(c, r, *p, s0);
+            r.s0 = a;
+            r.nsteps = nt;
+            r.dir = 1;
+            // from rest; its fields end with the launch, the strips' memories of tall threads live in d64
+            for (int j = 0; j < 8; ++j) r.psi[j] = *slot[5 + j];
+            r.lam = med[0]; r.mu = med[1]; r.muzx = med[2]; r.rhoz = med[3]; r.rhox = med[4];
+            r.zpf = d.zp;
+            r.xpf = d.xp;
+            r.src = src_args(c, s0 + a, ns);
+            r.rec = adj_args(c, s0 + a, ns);
+            r.seis_z = c->syn_z;
+            r.seis_x = c->syn_x;
+            HIPCHK(launch_resident_fp64(r, *p, c->N, ns, c->st));
+        }
+        resident_seismograms(c, s0, nb);
+        return FWI_OK;
+    }
     int isurf[4];
     for (int k = 0; k < 4; ++k) isurf[k] = c->g.isurf[k];
     for (int it = 0; it < nt; ++it) {
@@ -1482,6 +1659,16 @@ int setup_device(fwi_ctx *c, const fwi_acq *q) {
     c->surf_top_only = c->g.isurf[0] == N && c->g.isurf[1] == 0 && c->g.isurf[2] == 0 && c->g.isurf[3] == 0;
     for (int i = 0; c->fusable && i < c->nsrc_tot; ++i) c->fusable = interior(q->src_z[i], q->src_x[i]);
     for (int i = 0; c->fusable && i < c->nrec_tot; ++i) c->fusable = interior(q->rec_z[i], q->rec_x[i]);
+    {   // the resident propagation: cooperative launches, at most 2^16 - 2 points per shot list
+        HIPCHK(hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, c->o.device));
+        c->zmap_h = zmap;
+        c->xmap_h = xmap;
+        c->res_grid = c->fusable && c->nsrc_tot < 32767 && c->nrec_tot < 32767 && cooperative_ok(c->o.device, c->st);
+        if (c->res_grid) {
+            HIPCHK(hipHostMalloc((void **)&c->res_err, sizeof(int), hipHostMallocDefault));
+            *c->res_err = 0;
+        }
+    }
     RETIF(plan(c));
     RETIF(allocate(c));
     // snapshot cells outside the interior are never written by the one-pass step: zero once
@@ -1764,6 +1951,7 @@ void fwi_destroy(fwi_ctx *c) {
     }
     for (auto e : c->ev_pool) hipEventDestroy(e);
     free_all(c);
+    if (c->res_err) hipHostFree(c->res_err);
     if (c->st) hipStreamDestroy(c->st);
     delete c;
 }

@@ -220,6 +220,60 @@ void x_revcumsum(const double *adj_z, const double *adj_x, double *A_z, double *
 void x_media_chain(const XArgs &x, int nb, const double *mu, const double *rho, int z1, int z2, int x1, int x2,
                    double *d_lam, double *d_mu, double *d_rho, hipStream_t st);
 
+// ---- the resident propagation: many time steps in one launch (psv_resident.h) -----------
+// A tiling: shots per launch, tile size, tiles per shot, cells per thread, block and LDS size.
+struct ResPlan {
+    int shots, TX, TZ, ntx, ntz, cpt, threads;
+    int psi_lds, psi_rows, psi_cols;   // CPML memory in LDS: a tile's strip rows and columns, at most
+    size_t lds;
+};
+constexpr size_t kResLds = 160 * 1024;   // LDS of a CU
+// columns of a block's lanes (a tile is at most that wide) for a number of cells per thread
+constexpr int res_lanes(int cpt, int elt) { return cpt >= 4 && elt == 4 ? 64 : 32; }
+template <class T>
+struct ResArgs {
+    int nz, nx, P, nzs, nxs;
+    size_t fs;                          // nz * P
+    int shot0, s0;                      // the batch's first shot; the launch's first shot in the batch
+    int TX, TZ, ntx, ntz;
+    int psi_lds, psi_rows, psi_cols;
+    int t0, nsteps, dir, nt;            // time indices t0, t0 + dir, ...
+    T dt, cz[6], cx[6];
+    int load;                           // the state comes from and goes back to the arrays (else zero, dropped)
+    T *vz, *vx, *szz, *szx, *sxx, *uz, *ux, *We;   // [B][nz][P]
+    T *psi[8];                          // the order of pvz_z pvx_z pszz_z pszx_z, pvx_x pvz_x psxx_x pszx_x
+    const T *lam, *mu, *muzx, *rhoz, *rhox;        // [nz][P]
+    const CpmlPoint *zp, *xp;
+    const T *zpf, *xpf;                 // FP64: the profiles [nz][6], [nx][6]
+    int energy, surf;                   // We += v^2; row of a free surface at the top, or -1
+    int snap_z1, snap_z2, snap_x1, snap_x2, snap_dz, snap_dx, snap_dt, snz, snx;
+    int store, tb;                      // forward: snapshots from time index tb (slab 0) on; adjoint: slab 0's index
+    T *st[5];                           // vz vx szz szx sxx
+    size_t st_stride;
+    const T *sn[5];                     // adjoint: the same
+    size_t sn_stride;
+    T *g[5];                            // correlation sums [B][snz][snx], five with gform
+    double *g64;
+    size_t g64_stride;
+    int gform, flush_every;
+    T gw, gain_lm;
+    SrcArgs src, rec;                   // injected groups; recorded groups (ngroups 0: none)
+    double *seis_z, *seis_x;            // velocity samples, absolute rows [nt]
+    unsigned long long *mail;           // edge words, resident_words() of them
+    uint32_t epoch;                     // tag of the launch's first step
+    int *err;                           // host-visible: set when a wait gave up
+};
+// zmap, xmap: strip row / column of a grid line, -1 outside the strips
+bool plan_resident(int nz, int nx, int N, int nb, int elt, int cus, size_t lds, const std::vector<int> &zmap,
+                   const std::vector<int> &xmap, ResPlan *out);
+bool cooperative_ok(int device, hipStream_t st);
+size_t resident_words(const ResPlan &p, int N, int elt);
+hipError_t launch_resident_forward(const ResArgs<float> &r, const ResPlan &p, int N, int shots, hipStream_t st);
+hipError_t launch_resident_adjoint(const ResArgs<float> &r, const ResPlan &p, int N, int shots, hipStream_t st);
+hipError_t launch_resident_fp64(const ResArgs<double> &r, const ResPlan &p, int N, int shots, hipStream_t st);
+// urec2's running sums over rows of velocity samples [rows][nt], in place
+void launch_seis_scan(double *z, double *x, int rows, int nt, double dt, double dzdx, hipStream_t st);
+
 // ---- the FP64 propagation for seismograms (psv_fp64.hip) ------------------------------
 // The forward step of the exact path's kernels in FP64 (one thread per cell), with its own
 // FP64 media and CPML profiles, for the seismograms that the misfit and the adjoint
