@@ -26,7 +26,7 @@ LIB = PKG / "libfwi_psv.so"
 DRIVER = PKG / "fwi_psv"
 
 HIP_SOURCES = [  # the longest compiles first
-    "psv_resident_adj.hip", "psv_resident.hip", "psv_resident_f64.hip",
+    "psv_resident_adj.hip", "psv_resident.hip", "psv_resident_f64.hip", "psv_resident_exact.hip",
     "psv_step7_b.hip", "psv_step7_c.hip", "psv_step7.hip", "psv_stencil6.hip", "psv_v5.hip", "psv_v11.hip",
     "psv_v13.hip", "psv_kernels.hip", "psv_misc.hip", "psv_plain.hip", "psv_api.hip", "psv_noalloc.hip",
     "psv_exact.hip", "psv_fp64.hip"]

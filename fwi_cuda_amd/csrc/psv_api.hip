@@ -39,6 +39,9 @@ struct EventPair {
 
 size_t round_up(size_t v, size_t m) { return (v + m - 1) / m * m; }
 
+// workspace of the exact adjoint that a context keeps between calls, at most
+constexpr size_t kExactKeep = (size_t)8 << 30;
+
 // gain on the lam / mu correlation terms (divided out in FP64 on the host side)
 constexpr double kGainLM = 1152921504606846976.0;   // 2^60
 
@@ -144,16 +147,18 @@ struct fwi_ctx {
     int depth = 1; // rows the one-pass step loads ahead (autotuned)
     std::string tune_log;
 
-    // ---- the resident propagation (psv_resident.h): tilings per batch size, FP32 and FP64
+    // ---- the resident propagation (psv_resident.h): tilings per batch size
     // (shots 0: none), edge words, the next launch's first tag, flag of a wait that gave up
     bool res_grid = false;   // the grid, acquisition and device allow it
     int cus = 0;
     std::vector<int> zmap_h, xmap_h;
-    std::map<int, ResPlan> rplan, rplan64;
+    std::map<int, ResPlan> rplan[4];   // by ResKind
     unsigned long long *mail = nullptr;
     size_t mail_words = 0;
     uint32_t mail_tag = 1;
     int *res_err = nullptr;  // pinned host memory
+    char *xws = nullptr;     // the exact adjoint's workspace, kept while it is small (kExactKeep)
+    size_t xws_bytes = 0;
 
     // ---- profiling
     int prof_on = 0, prof_stride = 1;
@@ -436,22 +441,27 @@ RecArgs rec_args(fwi_ctx *c, int s0, int nb) {
 constexpr int kFlushSteps = 64;   // adjoint steps between flushes of the FP32 correlation sums
 
 // The tiling of the resident propagation for a batch of nb shots, or null where it does not
-// apply: a pinned kernel variant, rows or work order; a surface other than the top one at
-// row N, or a source or receiver outside the interior (the one-pass step's conditions); a
-// grid whose shot does not fit the chip's LDS.  Whether it applies does not depend on nb,
-// storage, graph replay or profiling: every pass of a context takes the same kernels.
-const ResPlan *resident_plan(fwi_ctx *c, int nb, bool fp64) {
-    if (!c->res_grid || c->plain || (!fp64 && (c->o.kernel_variant || c->o.tile_tz > 0 || c->o.work_order))) return nullptr;
-    auto &cache = fp64 ? c->rplan64 : c->rplan;
+// apply: a surface other than the top one at row N, or a source or receiver outside the
+// interior (the one-pass step's conditions); a grid whose shot does not fit the chip's LDS,
+// or whose steps the batched kernels run faster (plan_resident).  FP32 steps also keep to a
+// pinned kernel variant, rows per segment or work order; the FP64 propagation and the exact
+// adjoint's passes have no variants.
+enum ResKind { kResStep, kResFp64, kResExactForward, kResExact };
+const ResPlan *resident_plan(fwi_ctx *c, int nb, ResKind kind) {
+    if (!c->res_grid || c->plain) return nullptr;
+    if (kind == kResStep && (c->o.kernel_variant || c->o.tile_tz > 0 || c->o.work_order)) return nullptr;
+    auto &cache = c->rplan[kind];
     auto it = cache.find(nb);
     if (it == cache.end()) {
         ResPlan p{};
-        if (!plan_resident(c->g.nz, c->g.nx, c->N, nb, fp64 ? 8 : 4, c->cus, kResLds, c->zmap_h, c->xmap_h, &p)) p.shots = 0;
+        const ResUse use = kind == kResStep ? kUseStep : kind == kResFp64 ? kUseFp64 : kind == kResExact ? kUseExact
+                                                                                             : kUseExactForward;
+        if (!plan_resident(c->g.nz, c->g.nx, c->N, nb, use, c->cus, kResLds, c->zmap_h, c->xmap_h, &p)) p.shots = 0;
         it = cache.emplace(nb, p).first;
     }
     return it->second.shots > 0 ? &it->second : nullptr;
 }
-bool resident(fwi_ctx *c, int nb) { return resident_plan(c, nb, false) != nullptr; }
+bool resident(fwi_ctx *c, int nb) { return resident_plan(c, nb, kResStep) != nullptr; }
 
 // edge words for a tiling, and the first of n tags for a launch
 int resident_mail(fwi_ctx *c, const ResPlan &p, int elt, int n, uint32_t *tag) {
@@ -502,7 +512,7 @@ void resident_grid_args(const fwi_ctx *c, ResArgs<T> &r, const ResPlan &p, int s
 int resident_steps(fwi_ctx *c, int s0, int nb, const Wave &w, int t0, int nsteps, int dir, float *We, bool store,
                    int tb, bool record) {
     if (nsteps <= 0) return FWI_OK;
-    const ResPlan &p = *resident_plan(c, nb, false);
+    const ResPlan &p = *resident_plan(c, nb, kResStep);
     const bool adj = dir < 0;
     ResArgs<float> r{};
     for (int a = 0; a < nb; a += p.shots) {
@@ -1248,7 +1258,7 @@ int run_forward64(fwi_ctx *c, int s0, int nb) {
     HIPCHK(hipMemsetAsync(c->acc, 0, sizeof(double) * 2 * c->nrec_tot, c->st));
     const SrcArgs sa = src_args(c, s0, nb);
     const RecArgs ra = rec_args(c, s0, nb);
-    if (const ResPlan *p = resident_plan(c, nb, true)) {
+    if (const ResPlan *p = resident_plan(c, nb, kResFp64)) {
         ResArgs<double> r{};
         for (int a = 0; a < nb; a += p->shots) {
             const int ns = std::min(p->shots, nb - a);
@@ -1951,6 +1961,7 @@ void fwi_destroy(fwi_ctx *c) {
     }
     for (auto e : c->ev_pool) hipEventDestroy(e);
     free_all(c);
+    if (c->xws) hipFree(c->xws);
     if (c->res_err) hipHostFree(c->res_err);
     if (c->st) hipStreamDestroy(c->st);
     delete c;
@@ -2241,23 +2252,53 @@ int exact_gradient(fwi_ctx *c, int shot0, int nshots, const double *adj_z, const
         S = std::min(c->o.ckpt_interval, nt);
     else if (c->o.storage != FWI_STORE_FULL && per_shot_of(nt) + g_all > avail)
         S = std::max(1, std::min(nt, (int)std::lround(std::sqrt(13.0 * nt / 5.0))));
+    // The resident sweep takes no more shots at once, and no more steps per segment, than
+    // kExactKeep holds, and keeps that workspace for the next call: allocating and clearing
+    // the intermediates of all shots and steps anew takes longer than the sweep itself (301 x
+    // 601, 4 shots, 400 steps: 6.2 GB, 155 ms a call against 24), recomputing a segment's
+    // forward steps a fifth of it.
+    const bool res = resident_plan(c, 1, kResExact) && resident_plan(c, 1, kResExactForward);
+    size_t cap = avail;
+    if (res && c->o.storage != FWI_STORE_FULL) {
+        cap = std::min(avail, std::max(kExactKeep, g_all + per_shot_of(1)));
+        if (c->o.storage != FWI_STORE_CHECKPOINT || c->o.ckpt_interval <= 0) {
+            int nseg_ = 1;
+            while (per_shot_of((nt + nseg_ - 1) / nseg_) + g_all > cap && nseg_ < 64 && nseg_ < nt) ++nseg_;
+            S = std::min(S, (nt + nseg_ - 1) / nseg_);
+        }
+    }
     const size_t per_shot = per_shot_of(S);
     if (per_shot + g_all > avail)
         return c->fail(FWI_ENOMEM, "the exact adjoint keeps %.2f GB per shot (%d steps of intermediates), %.2f GB free",
                        per_shot / 1e9, S, avail / 1e9);
-    const int Bx = (int)std::min<size_t>((size_t)nshots, (avail - g_all) / per_shot);
+    const int Bx = (int)std::max<size_t>(
+        1, std::min<size_t>((size_t)nshots, cap > g_all ? (cap - g_all) / per_shot : 0));
     const int nseg = (nt + S - 1) / S;
-    std::vector<void *> mem;
-    auto A = [&](size_t bytes) -> void * {
-        void *p = nullptr;
-        if (hipMalloc(&p, bytes) != hipSuccess) return nullptr;
-        mem.push_back(p);
-        return p;
-    };
+    const size_t fl_bytes = sizeof(float) * fs * Bx * 30, hist_bytes = sizeof(float) * fs * Bx * 5 * (size_t)S,
+                 G_bytes = sizeof(double) * fs * 5 * nshots,
+                 ck_bytes = S < nt ? sizeof(float) * fs * Bx * 13 * (size_t)nseg : 0;
+    const size_t ws_bytes = fl_bytes + hist_bytes + G_bytes + ck_bytes;   // fs is a multiple of 64: aligned parts
+    if (ws_bytes > c->xws_bytes) {
+        if (c->xws) {
+            (void)hipStreamSynchronize(c->st);
+            (void)hipFree(c->xws);
+        }
+        c->xws = nullptr;
+        c->xws_bytes = 0;
+        if (hipMalloc((void **)&c->xws, ws_bytes) != hipSuccess) {
+            c->xws = nullptr;
+            (void)hipGetLastError();
+            return c->fail(FWI_ENOMEM, "exact adjoint buffers");
+        }
+        c->xws_bytes = ws_bytes;
+    }
+    // kept for the next call if it is small beside what is free, else given back
     auto release = [&]() {
         (void)hipStreamSynchronize(c->st);
-        for (void *p : mem) (void)hipFree(p);
-        mem.clear();
+        if (res && c->xws_bytes <= kExactKeep && c->xws_bytes <= freeb / 8) return;
+        (void)hipFree(c->xws);
+        c->xws = nullptr;
+        c->xws_bytes = 0;
     };
     XArgs x{};
     x.nz = nz; x.nx = nx; x.P = c->P; x.B = Bx; x.N = c->N;
@@ -2270,14 +2311,10 @@ int exact_gradient(fwi_ctx *c, int shot0, int nshots, const double *adj_z, const
     }
     x.lam = c->lam; x.mu = c->mu; x.muzx = c->muzx; x.rhoz = c->rhoz; x.rhox = c->rhox;
     x.zp = c->zp; x.xp = c->xp;
-    float *fl = static_cast<float *>(A(sizeof(float) * fs * Bx * 30));
-    float *hist = static_cast<float *>(A(sizeof(float) * fs * Bx * 5 * (size_t)S));
-    double *G = static_cast<double *>(A(sizeof(double) * fs * 5 * nshots));
-    float *ckp = S < nt ? static_cast<float *>(A(sizeof(float) * fs * Bx * 13 * (size_t)nseg)) : nullptr;
-    if (!fl || !hist || !G || (S < nt && !ckp)) {
-        release();
-        return c->fail(FWI_ENOMEM, "exact adjoint buffers");
-    }
+    float *fl = reinterpret_cast<float *>(c->xws);
+    float *hist = reinterpret_cast<float *>(c->xws + fl_bytes);
+    double *G = reinterpret_cast<double *>(c->xws + fl_bytes + hist_bytes);
+    float *ckp = S < nt ? reinterpret_cast<float *>(c->xws + fl_bytes + hist_bytes + G_bytes) : nullptr;
     float **slots[] = {&x.vz, &x.vx, &x.szz, &x.szx, &x.sxx, &x.pv[0], &x.pv[1], &x.pv[2], &x.pv[3],
                        &x.ps[0], &x.ps[1], &x.ps[2], &x.ps[3], &x.bvz, &x.bvx, &x.bzz, &x.bzx, &x.bxx,
                        &x.cv[0], &x.cv[1], &x.cv[2], &x.cv[3], &x.cs[0], &x.cs[1], &x.cs[2], &x.cs[3],
@@ -2321,6 +2358,79 @@ int exact_gradient(fwi_ctx *c, int shot0, int nshots, const double *adj_z, const
                                      hipMemcpyDeviceToDevice, c->st);
             }
         };
+        const ResPlan fp = res ? *resident_plan(c, nb, kResExactForward) : ResPlan{};
+        const ResPlan rp = res ? *resident_plan(c, nb, kResExact) : ResPlan{};
+        // steps [n0, n1) in one launch, with their intermediates if hist
+        auto res_forward = [&](int n0, int n1, bool with_hist) -> int {
+            ResArgs<float> q{};
+            for (int a = 0; a < nb; a += fp.shots) {
+                const int ns = std::min(fp.shots, nb - a);
+                RETIF(resident_mail(c, fp, 4, n1 - n0, &q.epoch));
+                resident_grid_args(c, q, fp, s0);
+                q.s0 = a;
+                q.t0 = n0; q.nsteps = n1 - n0; q.dir = 1;
+                q.load = 1;
+                q.vz = x.vz; q.vx = x.vx; q.szz = x.szz; q.szx = x.szx; q.sxx = x.sxx;
+                float *const psi[8] = {x.pv[0], x.pv[1], x.ps[0], x.ps[1], x.pv[3], x.pv[2], x.ps[3], x.ps[2]};
+                for (int j = 0; j < 8; ++j) q.psi[j] = psi[j];   // strip rows and columns only
+                q.lam = x.lam; q.mu = x.mu; q.muzx = x.muzx; q.rhoz = x.rhoz; q.rhox = x.rhox;
+                q.hist = with_hist ? x.hist : nullptr;
+                q.hist_base = n0;
+                q.hist_B = nb;
+                q.src = src_args(c, s0 + a, ns);
+                HIPCHK(launch_resident_forward(q, fp, c->N, ns, c->st));
+            }
+            return FWI_OK;
+        };
+        auto res_reverse = [&](int n0, int n1, const SrcArgs *type0) -> int {
+            ResExact q{};
+            q.nz = nz; q.nx = nx; q.P = c->P; q.nzs = c->nzs; q.nxs = c->nxs;
+            q.fs = fs;
+            q.shot0 = s0;
+            q.TX = rp.TX; q.TZ = rp.TZ; q.ntx = rp.ntx; q.ntz = rp.ntz;
+            q.psi_lds = rp.psi_lds; q.psi_rows = rp.psi_rows; q.psi_cols = rp.psi_cols;
+            q.t0 = n1 - 1; q.nsteps = n1 - n0;
+            q.dt = x.dt;
+            for (int k = 0; k < 6; ++k) q.cz[k] = x.cz[k], q.cx[k] = x.cx[k];
+            q.lam = x.lam; q.mu = x.mu; q.muzx = x.muzx; q.rhoz = x.rhoz; q.rhox = x.rhox;
+            q.zp = x.zp; q.xp = x.xp;
+            q.bvz = x.bvz; q.bvx = x.bvx; q.bzz = x.bzz; q.bzx = x.bzx; q.bxx = x.bxx;
+            float *const psi[8] = {x.cv[0], x.cv[1], x.cs[0], x.cs[1], x.cv[3], x.cv[2], x.cs[3], x.cs[2]};
+            for (int j = 0; j < 8; ++j) q.psi[j] = psi[j];
+            q.hist = x.hist;
+            q.hist_base = n0;
+            q.hist_B = nb;
+            q.surf = c->surf_top_only ? c->N : -1;
+            q.G = x.G;
+            q.err = c->res_err;
+            for (int a = 0; a < nb; a += rp.shots) {
+                const int ns = std::min(rp.shots, nb - a);
+                RETIF(resident_mail(c, rp, 4, n1 - n0, &q.epoch));
+                q.mail = c->mail;
+                q.s0 = a;
+                q.src = adj_args(c, s0 + a, ns);
+                q.rec = src_args(c, s0 + a, ns);
+                if (!type0) q.rec.ngroups = 0;
+                HIPCHK(launch_resident_exact(q, rp, c->N, ns, c->st));
+            }
+            return FWI_OK;
+        };
+        if (res) {
+            for (int k = 0; k < nseg && r == FWI_OK; ++k) {
+                if (S < nt) ckpt(k, true);
+                r = res_forward(k * S, std::min((k + 1) * S, nt), k == nseg - 1);
+            }
+            const SrcArgs *t0 = c->stf_type == 0 ? &fsa : nullptr;
+            for (int k = nseg - 1; k >= 0 && r == FWI_OK; --k) {
+                const int n0 = k * S, n1 = std::min(n0 + S, nt);
+                if (k < nseg - 1) {   // recompute the segment's intermediates from its checkpoint
+                    ckpt(k, false);
+                    r = res_forward(n0, n1, true);
+                }
+                if (r == FWI_OK) r = res_reverse(n0, n1, t0);
+            }
+            continue;
+        }
         // forward over all steps (each step's intermediates at its slot of the current
         // segment), saving the state at each segment start; the last segment's
         // intermediates are then in place for its reverse sweep
@@ -2360,8 +2470,7 @@ int exact_gradient(fwi_ctx *c, int shot0, int nshots, const double *adj_z, const
         x.G = G;
         x_media_chain(x, nshots, c->m_mu, c->m_rho, c->g.snap_z1, c->g.snap_z2, c->g.snap_x1, c->g.snap_x2, d_lam,
                       d_mu, d_rho, c->st);
-        const hipError_t e = hipStreamSynchronize(c->st);
-        if (e != hipSuccess) r = c->fail(FWI_EHIP, "exact adjoint: %s", hipGetErrorString(e));
+        r = sync(c);
     }
     release();
     return r;

@@ -18,7 +18,8 @@
 //   mu_zx += dt s'_zx e_zx                          rho_z^-1 += dt v'_z S_z,  rho_x^-1 likewise
 // plus the free-surface terms of the set stress 4 dt e (lam mu + mu^2) / (lam + 2 mu) and the
 // type-0 sources' inverse-density factor.  One thread per cell, every interior cell
-// stored: this path serves the autograd backward and its checks, not the FWI loop.
+// stored.  Grids that fit the chip's LDS, with the top free surface or none, take the
+// sweep of psv_resident_exact.hip instead.
 #include <algorithm>
 
 #include "psv_internal.h"

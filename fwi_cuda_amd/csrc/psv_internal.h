@@ -257,20 +257,46 @@ struct ResArgs {
     size_t g64_stride;
     int gform, flush_every;
     T gw, gain_lm;
+    T *hist;                            // forward: the exact adjoint's intermediates (XArgs::hist), or null
+    int hist_base, hist_B;
     SrcArgs src, rec;                   // injected groups; recorded groups (ngroups 0: none)
     double *seis_z, *seis_x;            // velocity samples, absolute rows [nt]
     unsigned long long *mail;           // edge words, resident_words() of them
     uint32_t epoch;                     // tag of the launch's first step
     int *err;                           // host-visible: set when a wait gave up
 };
+// What a tiling is for: FP32 steps, the FP64 propagation, the exact adjoint's two passes.
+enum ResUse { kUseStep, kUseFp64, kUseExactForward, kUseExact };
 // zmap, xmap: strip row / column of a grid line, -1 outside the strips
-bool plan_resident(int nz, int nx, int N, int nb, int elt, int cus, size_t lds, const std::vector<int> &zmap,
+bool plan_resident(int nz, int nx, int N, int nb, ResUse use, int cus, size_t lds, const std::vector<int> &zmap,
                    const std::vector<int> &xmap, ResPlan *out);
 bool cooperative_ok(int device, hipStream_t st);
 size_t resident_words(const ResPlan &p, int N, int elt);
 hipError_t launch_resident_forward(const ResArgs<float> &r, const ResPlan &p, int N, int shots, hipStream_t st);
 hipError_t launch_resident_adjoint(const ResArgs<float> &r, const ResPlan &p, int N, int shots, hipStream_t st);
 hipError_t launch_resident_fp64(const ResArgs<double> &r, const ResPlan &p, int N, int shots, hipStream_t st);
+// The exact adjoint's reverse sweep (psv_exact.hip's step) over time indices t0, t0 - 1, ...
+struct ResExact {
+    int nz, nx, P, nzs, nxs;
+    size_t fs;
+    int shot0, s0;
+    int TX, TZ, ntx, ntz;
+    int psi_lds, psi_rows, psi_cols;
+    int t0, nsteps;
+    float dt, cz[6], cx[6];
+    const float *lam, *mu, *muzx, *rhoz, *rhox;
+    const CpmlPoint *zp, *xp;
+    float *bvz, *bvx, *bzz, *bzx, *bxx;   // adjoint state [B][nz][P]
+    float *psi[8];                        // carries: z strips cv0 cv1 cs0 cs1, x strips cv3 cv2 cs3 cs2
+    const float *hist;
+    int hist_base, hist_B, surf;
+    double *G;                            // [B][5][nz][P]
+    SrcArgs src, rec;                     // receivers' adjoint sources; type-0 sources (ngroups 0: none)
+    unsigned long long *mail;
+    uint32_t epoch;
+    int *err;
+};
+hipError_t launch_resident_exact(const ResExact &r, const ResPlan &p, int N, int shots, hipStream_t st);
 // urec2's running sums over rows of velocity samples [rows][nt], in place
 void launch_seis_scan(double *z, double *x, int rows, int nt, double dt, double dzdx, hipStream_t st);
 

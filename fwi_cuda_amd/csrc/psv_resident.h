@@ -203,7 +203,8 @@ __device__ __forceinline__ double prof_at(const ResArgs<double> &, const CpmlPoi
 template <class T, int N, int CPT, int LX, bool ADJ>
 __global__ __launch_bounds__(1024) void k_resident(const ResArgs<T> r) {
     extern __shared__ char smem[];
-    constexpr bool kReg = CPT <= 2;             // gradient sums in registers, edges published by their owners
+    constexpr bool kReg = CPT <= 2;             // gradient sums in registers
+    constexpr bool kOwn = CPT <= 4;             // edges published by their owners
     // CPML memory: in registers where they hold it, else in LDS (r.psi_lds) or the arrays
     constexpr bool kPsiReg = CPT * (int)sizeof(T) * (ADJ ? 2 : 1) <= 8;
     constexpr int QL = CPT + 2 * N - 1;         // rows a thread's z taps span
@@ -443,6 +444,15 @@ __global__ __launch_bounds__(1024) void k_resident(const ResArgs<T> r) {
                     vx_x = vx_x * xk + p1;
                     vz_x = vz_x * xkh + p2;
                 }
+                if constexpr (!ADJ && sizeof(T) == 4) {   // the strain rates the reverse sweep reads
+                    if (r.hist && k < nc) {
+                        T *hp = res_seg<T>()->hist + ((size_t)(it - r.hist_base) * r.hist_B + s) * 5 * r.fs +
+                                (uint32_t)((z0 + zv + k) * r.P + ix);
+                        hp[0] = vz_z;
+                        hp[r.fs] = vx_x;
+                        hp[2 * r.fs] = vz_x + vx_z;
+                    }
+                }
                 const T l = lam[k], m = mu[k];
                 const T div = l * (vx_x + vz_z);
                 T nzz = lzz[c] + dt * (div + T(2) * m * vz_z);
@@ -456,11 +466,11 @@ __global__ __launch_bounds__(1024) void k_resident(const ResArgs<T> r) {
                 lzz[c] = nzz;
                 lzx[c] = nzx;
                 lxx[c] = nxx;
-                if constexpr (!kReg) __builtin_amdgcn_sched_barrier(0);
-                if constexpr (kReg) ed.publish(res_seg<T>()->mail + ed.ph, tag, zv + k, xv, nzz, nzx, nzx, nxx);
+                if constexpr (CPT > 2) __builtin_amdgcn_sched_barrier(0);
+                if constexpr (kOwn) ed.publish(res_seg<T>()->mail + ed.ph, tag, zv + k, xv, nzz, nzx, nzx, nxx);
             }
         }
-        if constexpr (!kReg) {
+        if constexpr (!kOwn) {
             lds_barrier();
             publish_runs(true, tag);
         }
@@ -514,6 +524,14 @@ __global__ __launch_bounds__(1024) void k_resident(const ResArgs<T> r) {
                     sxx_x = sxx_x * xk + p1;
                     szx_x = szx_x * xkh + p2;
                 }
+                if constexpr (!ADJ && sizeof(T) == 4) {   // the stress divergences
+                    if (r.hist && k < nc) {
+                        T *hp = res_seg<T>()->hist + (((size_t)(it - r.hist_base) * r.hist_B + s) * 5 + 3) * r.fs +
+                                (uint32_t)((z0 + zv + k) * r.P + ix);
+                        hp[0] = szx_x + szz_z;
+                        hp[r.fs] = sxx_x + szx_z;
+                    }
+                }
                 const T vz0 = lvz[c], vx0 = lvx[c];
                 const T vz1 = vz0 + dt * rhoz[k] * (szx_x + szz_z);
                 const T vx1 = vx0 + dt * rhox[k] * (sxx_x + szx_z);
@@ -524,24 +542,33 @@ __global__ __launch_bounds__(1024) void k_resident(const ResArgs<T> r) {
                 if (r.energy) we[k] = we[k] + (vx1 * vx1 + vz1 * vz1);
                 lvz[c] = vz1;
                 lvx[c] = vx1;
-                if constexpr (!kReg) __builtin_amdgcn_sched_barrier(0);
+                if constexpr (CPT > 2) __builtin_amdgcn_sched_barrier(0);
             }
         }
         if constexpr (ADJ) {
             if (gstep && lat) {                 // fwi_grad2 (:439-484)
                 const RSeg<T> q = res_seg<T>();
+                // a thread of many cells reads all its slab cells and sums first: one latency
+                T S[5][CPT], gm[kReg ? 1 : 5][CPT];
+                int lc[CPT];
+#pragma unroll
+                for (int k = 0; k < CPT; ++k) {
+                    lc[k] = lat >> k & 1 ? lat_cell(zv + k) : 0;
+#pragma unroll
+                    for (int j = 0; j < 5; ++j) {
+                        if constexpr (kReg) {
+                            S[j][k] = sn[j][k];
+                        } else {
+                            S[j][k] = q->sn[j][snoff + lc[k]];
+                            gm[j][k] = j < ng ? q->g[j][(size_t)s * slab + lc[k]] : T(0);
+                        }
+                    }
+                }
 #pragma unroll
                 for (int k = 0; k < CPT; ++k) {
                     if (!(lat >> k & 1)) continue;
                     const int c = base + k * W;
-                    const int lc = lat_cell(zv + k);
-                    T S[5];
-#pragma unroll
-                    for (int j = 0; j < 5; ++j) {
-                        if constexpr (kReg) S[j] = sn[j][k];
-                        else S[j] = q->sn[j][snoff + lc];
-                    }
-                    const T Vz = S[0], Vx = S[1], Szz = S[2], Szx = S[3], Sxx = S[4];
+                    const T Vz = S[0][k], Vx = S[1][k], Szz = S[2][k], Szx = S[3][k], Sxx = S[4][k];
                     const T c_zz = lzz[c], c_xx = lxx[c], c_zx = lzx[c];
                     const T lm = lam[k] + mu[k];
                     const T il = r.gain_lm / (lm * lm), im = r.gain_lm / (mu[k] * mu[k]);
@@ -549,12 +576,8 @@ __global__ __launch_bounds__(1024) void k_resident(const ResArgs<T> r) {
                     const T s2 = T(0.25) * im * (Szz - Sxx) * (c_zz - c_xx);
                     const T s3 = im * (Szx * c_zx);
                     auto add = [&](int j, T v) {
-                        if constexpr (kReg) {
-                            gs[j][k] = gs[j][k] + r.gw * v;
-                        } else {
-                            T *g = q->g[j] + ((size_t)s * slab + lc);
-                            *g = *g + r.gw * v;
-                        }
+                        if constexpr (kReg) gs[j][k] = gs[j][k] + r.gw * v;
+                        else q->g[j][(size_t)s * slab + lc[k]] = gm[j][k] + r.gw * v;
                     };
                     add(0, s1);
                     if (!r.gform) {
@@ -603,7 +626,7 @@ __global__ __launch_bounds__(1024) void k_resident(const ResArgs<T> r) {
             }
         }
         if (n + 1 < r.nsteps) {
-            if constexpr (kReg) {
+            if constexpr (kOwn) {
                 if (act)
 #pragma unroll
                     for (int k = 0; k < CPT; ++k) {

@@ -45,15 +45,26 @@ int strip_lines(const std::vector<int> &map, int N, int T) {
     return most;
 }
 
+}  // namespace
+
 // The tiling that takes the least time for nb shots on cus compute units with lds bytes each,
-// by a model of a launch's step in us: its barriers and latencies, the two edge exchanges,
-// the cells of a thread (a chain) and of the block (issue), the edge values.  Every tile
-// holds at least N rows and columns (its halo comes from direct neighbours only).
-bool plan_tiles(int nz, int nx, int N, int nb, int elt, int fields, int max_cpt, int cus, size_t lds,
-                const std::vector<int> &zmap, const std::vector<int> &xmap, ResPlan *out) {
+// by measured step times in us: a base (the barriers and latencies of the chain of a thread's
+// cells, and the two edge exchanges) and a slope per lane-cell of the block.  One cell per
+// thread: 3.8 at 300 cells, 4.4 at 740; two: 5.6 at 450, 6.5 at 1600; four: 10.8 at 3300;
+// eight (its registers spill): 25 at 4600.  FP64 and the exact adjoint's sweep cost what
+// their registers and words do; that sweep with four cells per thread spills its FP64 sums
+// (301 x 601, 4 shots: 31 us a step against 2 x 10 for two launches of two cells per
+// thread).  Every tile holds at least N rows and columns (its halo comes from direct
+// neighbours only).  FP32 steps that the batched kernels run as fast, at 16 us of launches
+// and 14.4 us per million cells, are left to them: 600 x 1100, 8 shots take 78 us there and
+// 82 here, 800 x 1400, 1 shot 35 and 26.
+bool plan_resident(int nz, int nx, int N, int nb, ResUse use, int cus, size_t lds, const std::vector<int> &zmap,
+                   const std::vector<int> &xmap, ResPlan *out) {
+    const int elt = use == kUseFp64 ? 8 : 4, fields = use == kUseExact ? 4 : 5;
+    const int max_cpt = use == kUseStep || use == kUseExactForward ? 8 : 4;
     const int iz = nz - 2 * N, ix = nx - 2 * N;
     double best = 1e300;
-    const double e = elt / 4.0;
+    const double e = use == kUseFp64 ? 1.8 : use == kUseExact ? 1.5 : 1.0;
     for (int g = 1; g <= std::min(nb, cus); ++g) {
         const int launches = (nb + g - 1) / g, tiles = cus / g;
         if (g > 1 && (nb + g - 2) / (g - 1) == launches) continue;   // fewer shots a launch, as many launches
@@ -72,8 +83,10 @@ bool plan_tiles(int nz, int nx, int N, int nb, int elt, int fields, int max_cpt,
                     if (thr > 1024 || need > lds) continue;
                     const int items = (ntz > 1 ? 4 * N * TX : 0) + (ntx > 1 ? 4 * N * TZ : 0);
                     if (items > kResItems * thr) continue;
-                    const bool alone = ntx * ntz == 1;
-                    double t = 1.0 + (alone ? 0.0 : 2.2) + 0.2 * cpt * e + 1.6e-3 * e * TX * TZ + 0.25e-3 * e * items;
+                    const double base = cpt == 1 ? 3.5 : cpt == 2 ? 5.0 : cpt == 4 ? 5.2 : 7.0;
+                    const double slope = cpt <= 2 ? 0.9e-3 : cpt == 4 ? (use == kUseExact ? 3e-3 : 1.75e-3) : 3.9e-3;
+                    double t = base - (ntx * ntz == 1 ? 2.4 : 0.0) + e * slope * res_lanes(cpt, elt) * TZ +
+                               e * 0.25e-3 * items;
                     const int srows = strip_lines(zmap, N, TZ);
                     const size_t psi = (size_t)4 * elt * (srows * TX + cols * TZ);
                     const bool psi_lds = need + psi <= lds;
@@ -86,13 +99,7 @@ bool plan_tiles(int nz, int nx, int N, int nb, int elt, int fields, int max_cpt,
                 }
         }
     }
-    return best < 1e299;
-}
-
-}  // namespace
-
-void launch_seis_scan(double *z, double *x, int rows, int nt, double dt, double dzdx, hipStream_t st) {
-    if (rows > 0) hipLaunchKernelGGL(k_seis_scan, dim3(rows, 2), dim3(64), 0, st, z, x, nt, dt, dzdx);
+    return best < (use == kUseStep ? 0.9 * (16.0 + 14.4e-6 * nb * nz * nx) : 1e299);
 }
 
 // Cooperative launches work: the attribute, and one empty launch (the runtime's cooperative
@@ -107,9 +114,8 @@ bool cooperative_ok(int device, hipStream_t st) {
     return true;
 }
 
-bool plan_resident(int nz, int nx, int N, int nb, int elt, int cus, size_t lds, const std::vector<int> &zmap,
-                   const std::vector<int> &xmap, ResPlan *out) {
-    return plan_tiles(nz, nx, N, nb, elt, 5, elt == 8 ? 4 : 8, cus, lds, zmap, xmap, out);
+void launch_seis_scan(double *z, double *x, int rows, int nt, double dt, double dzdx, hipStream_t st) {
+    if (rows > 0) hipLaunchKernelGGL(k_seis_scan, dim3(rows, 2), dim3(64), 0, st, z, x, nt, dt, dzdx);
 }
 
 size_t resident_words(const ResPlan &p, int N, int elt) {
