@@ -63,7 +63,9 @@ struct fwi_ctx {
     double step_est = 0.01;
 
     // ---- plan
-    int B = 1, storage = FWI_STORE_FULL, S = 0, nseg = 0;
+    int B = 1;    // shots whose fields fit: a batch of forward passes
+    int Bg = 1;   // shots of a gradient's batch (snapshots, sums), at most B
+    int storage = FWI_STORE_FULL, S = 0, nseg = 0;
     // CHECKPOINT: nseg units of S steps and `slots` checkpoint buffers; with slots < nseg - 1
     // the reversal advances from held states on a binomial schedule (ck_top / ck_rev: best
     // split of a chain of n units with s free slots, index n * (slots + 1) + s)
@@ -142,6 +144,7 @@ struct fwi_ctx {
     bool plain = false;
     PlainBufs pb{};
     bool tuned = false;
+    int tuned_nb = 0;   // the batch it was tuned for
     int var = 2;   // stencil kernel variant (autotuned); 4 = one-pass step
     int order = 0; // stencil work order (autotuned)
     int depth = 1; // rows the one-pass step loads ahead (autotuned)
@@ -372,7 +375,7 @@ KArgs base_args(fwi_ctx *c, int nb, const Wave &w) {
     a.g_rho = c->gr[2];
     a.gform = c->gform;
     a.g_ext = c->gx;
-    a.g_ext_stride = (size_t)c->B * c->snz * c->snx;
+    a.g_ext_stride = (size_t)c->Bg * c->snz * c->snx;
     a.gw = (float)(c->o.grad_sign * (double)c->g.snap_dt * c->g.dt);
     a.gain_lm = (float)kGainLM;
     a.order = c->order;
@@ -531,7 +534,7 @@ int resident_steps(fwi_ctx *c, int s0, int nb, const Wave &w, int t0, int nsteps
         r.tb = tb;
         for (int j = 0; j < 5; ++j) r.st[j] = c->snap[j], r.sn[j] = c->snap[j];
         r.st_stride = r.sn_stride = c->snap_stride;
-        const size_t cells = (size_t)c->B * c->snz * c->snx;
+        const size_t cells = (size_t)c->Bg * c->snz * c->snx;
         float *g[5] = {c->gr[0], c->gr[1], c->gr[2], c->gx, c->gx + cells};
         for (int j = 0; j < 5; ++j) r.g[j] = g[j];
         r.g64 = c->gr64;
@@ -728,7 +731,7 @@ int ckpt_copy(fwi_ctx *c, int k, int nb, const Wave &w, bool save) {
         void *dst = save ? (void *)(base + off) : (void *)p;
         const void *src = save ? (const void *)p : (const void *)(base + off);
         HIPCHK(hipMemcpyAsync(dst, src, nbytes, hipMemcpyDeviceToDevice, c->st));
-        off += sizeof(float) * per * c->B;
+        off += sizeof(float) * per * c->Bg;
     }
     return FWI_OK;
 }
@@ -750,8 +753,9 @@ int check_finite(fwi_ctx *c, int nb) {
 // the best is kept per (grid, order, batch) for the process.
 struct TuneKey {
     int nz, nx, N, B;
+    bool fwd;
     bool operator<(const TuneKey &o) const {
-        return std::tie(nz, nx, N, B) < std::tie(o.nz, o.nx, o.N, o.B);
+        return std::tie(nz, nx, N, B, fwd) < std::tie(o.nz, o.nx, o.N, o.B, o.fwd);
     }
 };
 struct TuneVal {
@@ -760,17 +764,21 @@ struct TuneVal {
 std::map<TuneKey, TuneVal> g_tuned;
 std::mutex g_tune_mu;
 
-void take(fwi_ctx *c, const TuneVal &v) {
+void take(fwi_ctx *c, const TuneVal &v, int nb) {
     c->var = v.var;
     c->tz = v.tz;
     c->depth = v.depth;
     c->order = v.order;
     c->tuned = true;
+    c->tuned_nb = nb;
 }
 
 int autotune(fwi_ctx *c, int nb) {
-    if (c->plain || c->tuned || resident(c, nb)) return FWI_OK;
-    const TuneKey key{c->g.nz, c->g.nx, c->N, nb};
+    if (c->plain || resident(c, nb) || (c->tuned && c->tuned_nb == nb)) return FWI_OK;
+    // a forward batch larger than a gradient's is tuned by forward steps alone: snapshots and
+    // sums hold a gradient's batch only
+    const bool fwd = nb > c->Bg;
+    const TuneKey key{c->g.nz, c->g.nx, c->N, nb, fwd};
     const int fv = c->o.kernel_variant;   // 0 = any
     const bool order_forced = c->o.work_order >= 1 && c->o.work_order <= 4;
     // candidates (variant, rows per segment, prefetch depth); the one-pass step only where it applies
@@ -808,7 +816,7 @@ int autotune(fwi_ctx *c, int nb) {
                                    "variant 4's conditions and variant 6's z CPML strips)"
                                  : "");
     if (cand.size() == 1 && order_forced) {   // nothing left to choose
-        take(c, {cand[0].var, cand[0].tz, cand[0].depth, c->o.work_order - 1});
+        take(c, {cand[0].var, cand[0].tz, cand[0].depth, c->o.work_order - 1}, nb);
         return FWI_OK;
     }
     {
@@ -817,7 +825,7 @@ int autotune(fwi_ctx *c, int nb) {
         if (it != g_tuned.end() && (!fv || fv == it->second.var) && (!one_pass(it->second.var) || c->fusable) &&
             (!order_forced || c->o.work_order - 1 == it->second.order) &&
             (c->o.tile_tz <= 0 || c->o.tile_tz == it->second.tz)) {
-            take(c, it->second);
+            take(c, it->second, nb);
             return FWI_OK;
         }
     }
@@ -850,8 +858,8 @@ int autotune(fwi_ctx *c, int nb) {
     ap.displ = 1;
     std::vector<KArgs *> mix;
     for (int k = 0; k < kmix; ++k) mix.push_back(&a);
-    for (int k = 0; k < kmix; ++k) mix.push_back(k ? &ar : &as);
-    for (int k = 0; k < kmix; ++k) mix.push_back(k ? &ap : &ag);
+    for (int k = 0; k < kmix && !fwd; ++k) mix.push_back(k ? &ar : &as);
+    for (int k = 0; k < kmix && !fwd; ++k) mix.push_back(k ? &ap : &ag);
     auto run = [&](const TuneVal &v) {
         for (KArgs *x : mix) {
             x->order = a.order;
@@ -889,7 +897,7 @@ int autotune(fwi_ctx *c, int nb) {
     }
     hipEventDestroy(e0);
     hipEventDestroy(e1);
-    take(c, bv);
+    take(c, bv, nb);
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tuned[key] = bv;
     return FWI_OK;
@@ -1005,7 +1013,7 @@ bool flush_after(int nt, int it) { return (nt - it) % kFlushSteps == 0; }
 // the batch's FP32 correlation sums added into their FP64 totals and zeroed
 void flush_sums(fwi_ctx *c, int nb) {
     Timer t(c, FWI_K_OTHER);
-    const size_t cells = (size_t)c->B * c->snz * c->snx;
+    const size_t cells = (size_t)c->Bg * c->snz * c->snx;
     float *g[5] = {c->gr[0], c->gr[1], c->gr[2], c->gx, c->gx + cells};
     dev_flush_sums(c->gr64, g, c->gform ? 5 : 3, (size_t)nb * c->snz * c->snx, cells, c->st);
 }
@@ -1013,7 +1021,7 @@ void flush_sums(fwi_ctx *c, int nb) {
 // the same inside a captured chunk of adjoint steps: step k of the chunk is time index
 // *si_base - k, known only at replay, so the kernel itself decides whether to flush
 void flush_sums_at(fwi_ctx *c, int nb, int k) {
-    const size_t cells = (size_t)c->B * c->snz * c->snx;
+    const size_t cells = (size_t)c->Bg * c->snz * c->snx;
     float *g[5] = {c->gr[0], c->gr[1], c->gr[2], c->gx, c->gx + cells};
     dev_flush_sums_at(c->gr64, g, c->gform ? 5 : 3, (size_t)nb * c->snz * c->snx, cells, c->si_base, -1, k,
                       c->g.nt, kFlushSteps, c->st);
@@ -1028,8 +1036,8 @@ int run_adjoint(fwi_ctx *c, int s0, int nb) {
     HIPCHK(hipMemsetAsync(c->f[8], 0, sizeof(float) * nb * c->fs(), c->st));
     for (int i = 0; i < 3; ++i)
         HIPCHK(hipMemsetAsync(c->gr[i], 0, sizeof(float) * nb * c->snz * c->snx, c->st));
-    if (c->gform) HIPCHK(hipMemsetAsync(c->gx, 0, sizeof(float) * 2 * c->B * c->snz * c->snx, c->st));
-    HIPCHK(hipMemsetAsync(c->gr64, 0, sizeof(double) * 5 * c->B * c->snz * c->snx, c->st));
+    if (c->gform) HIPCHK(hipMemsetAsync(c->gx, 0, sizeof(float) * 2 * c->Bg * c->snz * c->snx, c->st));
+    HIPCHK(hipMemsetAsync(c->gr64, 0, sizeof(double) * 5 * c->Bg * c->snz * c->snx, c->st));
     KArgs a = base_args(c, nb, w);
     a.We = c->f[8];
     a.energy = 1;
@@ -1213,10 +1221,10 @@ int absmax_host(fwi_ctx *c, const double *x, size_t n, double *out) {
     return sync(c);
 }
 
-int batches(const fwi_ctx *c, int shot0, int nshots, std::vector<std::pair<int, int>> &out) {
+int batches(const fwi_ctx *c, int shot0, int nshots, int B, std::vector<std::pair<int, int>> &out) {
     out.clear();
     if (shot0 < 0 || nshots < 0 || shot0 + nshots > c->nshot) return FWI_EINVAL;
-    const int nbat = (nshots + c->B - 1) / c->B;
+    const int nbat = (nshots + B - 1) / B;
     for (int b = 0, s = shot0; b < nbat; ++b) {
         const int left = shot0 + nshots - s, rem = nbat - b;
         const int nb = (left + rem - 1) / rem;   // balanced batches
@@ -1333,6 +1341,7 @@ int refresh_media(fwi_ctx *c) {
 // ---------------------------------------------------------------------------
 struct Need {
     size_t shared, per_shot, per_shot_fp64;
+    size_t per_shot_grad;   // the part of per_shot that only a gradient's batch takes
 };
 
 Need need_bytes(const fwi_ctx *c, int storage, int S, int slots, int keep = 1) {
@@ -1347,18 +1356,19 @@ Need need_bytes(const fwi_ctx *c, int storage, int S, int slots, int keep = 1) {
         n.per_shot_fp64 = 15 * fs * 8;
     }
     const size_t state_ck = 5 * fs * 4 + 4 * (c->psiz() + c->psix()) * 4;
-    n.per_shot = 9 * fs * 4 + 8 * (c->psiz() + c->psix()) * 4 + 5 * snapcell * 4 + 5 * snapcell * 8 +
-                 n.per_shot_fp64;
+    n.per_shot = 9 * fs * 4 + 8 * (c->psiz() + c->psix()) * 4 + n.per_shot_fp64;
+    n.per_shot_grad = 5 * snapcell * 4 + 5 * snapcell * 8;
     if (c->plain) n.per_shot += 12 * fs * 4;
     // second time level of the one-pass step (5 fields, 4 stress-side psi)
     const size_t level2 = c->fusable ? (5 * fs + 2 * (c->psiz() + c->psix())) * 4 : 0;
     n.per_shot += level2;
     if (storage == FWI_STORE_FULL) {
-        n.per_shot += 5 * (size_t)c->snt * snapcell * 4;
+        n.per_shot_grad += 5 * (size_t)c->snt * snapcell * 4;
     } else {
-        n.per_shot += state_ck + level2 + (size_t)slots * state_ck +
+        n.per_shot_grad += state_ck + level2 + (size_t)slots * state_ck +
                       (size_t)std::max(keep, 1) * 5 * (size_t)(S / c->g.snap_dt) * snapcell * 4;
     }
+    n.per_shot += n.per_shot_grad;
     return n;
 }
 
@@ -1398,6 +1408,47 @@ long long plan_schedule(int n, int s, std::vector<int> &top_m, std::vector<int> 
 }
 
 constexpr int kMaxUnits = 2048;   // the schedule's dynamic programme is O(units^2 slots)
+
+// The shots of a gradient's batch and its storage, where the caller leaves both open: a step
+// of all shots costs each pass's launches (16 us a batch) and cells (forward and adjoint 33
+// us per million, a recomputed step 12 more), and a smaller batch recomputes less or
+// nothing.  The fields still hold c->B shots, for forward passes.  Measured per gradient:
+// 1001 x 2001, 8 shots, 480 steps in 24 GB 374 ms as one checkpointed batch, 324 as two
+// full ones; 2001 x 4001, 2 shots, 240 steps in 16 GB 224 and 195.
+int plan_gradient_batch(fwi_ctx *c, int storage, int S, int slots, int units, size_t budget) {
+    const double cells = 1e-6 * c->g.nz * c->g.nx * c->nshot;
+    // recomputed share of the steps with batches of b shots, or -1 if they do not fit
+    auto recomputed = [&](int st, int b) -> double {
+        const Need n = need_bytes(c, st, S, slots, 1);
+        const size_t fixed = n.shared + (size_t)c->B * (n.per_shot - n.per_shot_grad);
+        if (fixed + (size_t)b * n.per_shot_grad > budget) return -1.0;
+        if (st == FWI_STORE_FULL) return 0.0;
+        if (units < 2) return 0.0;
+        const Need k = need_bytes(c, st, S, slots - 1, 2);
+        if (k.per_shot_grad <= n.per_shot_grad) return 0.0;
+        const size_t more = (budget - fixed - (size_t)b * n.per_shot_grad) / ((size_t)b * (k.per_shot_grad - n.per_shot_grad));
+        return std::max(0.0, (double)(units - 1) - (double)more) * S / c->g.nt;
+    };
+    auto cost = [&](int st, int b) {
+        const double rf = recomputed(st, b);
+        const int nbat = (c->nshot + b - 1) / b;
+        return rf < 0 ? 1e300 : nbat * 16.0 * (2.0 + rf) + cells * (33.0 + 12.0 * rf);
+    };
+    double best = 0.97 * cost(storage, c->B);   // a change has to be worth it
+    int st = storage;
+    for (int nbat = (c->nshot + c->B - 1) / c->B, last = 0; nbat <= c->nshot; ++nbat) {
+        const int b = (c->nshot + nbat - 1) / nbat;
+        if (b == last) continue;
+        last = b;
+        for (int s : {(int)FWI_STORE_FULL, (int)FWI_STORE_CHECKPOINT})
+            if (cost(s, b) < best) {
+                best = cost(s, b);
+                c->Bg = b;
+                st = s;
+            }
+    }
+    return st;
+}
 
 int plan(fwi_ctx *c) {
     size_t freeb = 0, total = 0;
@@ -1479,7 +1530,10 @@ int plan(fwi_ctx *c) {
     if (c->plain) Bmax = 1;
     Bmax = std::max(1, Bmax);
     const int nbat = (c->nshot + Bmax - 1) / Bmax;
-    c->B = (c->nshot + nbat - 1) / nbat;
+    c->B = c->Bg = (c->nshot + nbat - 1) / nbat;
+    if (c->o.storage == FWI_STORE_AUTO && c->o.batch <= 0 && c->o.ckpt_interval <= 0 && c->o.ckpt_slots <= 0 &&
+        c->o.ckpt_keep <= 0 && !c->plain && slots >= units_of(S) - 1)
+        storage = plan_gradient_batch(c, storage, S, slots, units_of(S), budget);
     c->storage = storage;
     c->S = S;
     c->nseg = units_of(S);
@@ -1496,11 +1550,12 @@ int plan(fwi_ctx *c) {
         const int cap = c->o.ckpt_keep > 0 ? std::min(c->o.ckpt_keep, c->nseg) : c->nseg;
         if (cap > 1 && slots >= c->nseg - 1) {
             const Need k1 = need_bytes(c, storage, S, slots, 1), k2 = need_bytes(c, storage, S, slots - 1, 2);
-            const size_t used = k1.shared + (size_t)c->B * k1.per_shot;
+            const size_t used = k1.shared + (size_t)c->B * (k1.per_shot - k1.per_shot_grad) +
+                                (size_t)c->Bg * k1.per_shot_grad;
             if (k2.per_shot <= k1.per_shot) {
                 keep = cap;
             } else if (used <= budget) {
-                const size_t more = (budget - used) / ((size_t)c->B * (k2.per_shot - k1.per_shot));
+                const size_t more = (budget - used) / ((size_t)c->Bg * (k2.per_shot - k1.per_shot));
                 keep = (int)std::min<size_t>((size_t)cap, 1 + more);
             }
         }
@@ -1524,7 +1579,7 @@ int plan(fwi_ctx *c) {
 }
 
 int allocate(fwi_ctx *c) {
-    const int nz = c->g.nz, nx = c->g.nx, nt = c->g.nt, B = c->B;
+    const int nz = c->g.nz, nx = c->g.nx, nt = c->g.nt, B = c->B, Bg = c->Bg;
     const size_t fs = c->fs(), nn = (size_t)nz * nx, snapcell = (size_t)c->snz * c->snx;
     bool ok = true;
     auto F = [&](size_t n) { float *p = c->dalloc<float>(n); ok = ok && p; return p; };
@@ -1561,28 +1616,28 @@ int allocate(fwi_ctx *c) {
     for (int i = 0; i < 9; ++i) c->f[i] = F(B * fs);
     for (int i = 0; i < 4; ++i) c->psi[i] = F(B * c->psiz());
     for (int i = 4; i < 8; ++i) c->psi[i] = F(B * c->psix());
-    for (int i = 0; i < 3; ++i) c->gr[i] = F(B * snapcell);
-    c->gx = F(2 * B * snapcell);
-    c->gr64 = D(5 * (size_t)B * snapcell);
-    auto level2 = [&](float **f2, float **psi2) {
-        for (int i = 0; i < 5; ++i) f2[i] = F(B * fs);
-        for (int i = 0; i < 2; ++i) psi2[i] = F(B * c->psiz());
-        for (int i = 2; i < 4; ++i) psi2[i] = F(B * c->psix());
+    for (int i = 0; i < 3; ++i) c->gr[i] = F(Bg * snapcell);
+    c->gx = F(2 * Bg * snapcell);
+    c->gr64 = D(5 * (size_t)Bg * snapcell);
+    auto level2 = [&](float **f2, float **psi2, int n) {
+        for (int i = 0; i < 5; ++i) f2[i] = F(n * fs);
+        for (int i = 0; i < 2; ++i) psi2[i] = F(n * c->psiz());
+        for (int i = 2; i < 4; ++i) psi2[i] = F(n * c->psix());
     };
-    if (c->fusable) level2(c->f2, c->psi2);
+    if (c->fusable) level2(c->f2, c->psi2, B);
     if (c->storage == FWI_STORE_FULL) {
         c->snap_stride = (size_t)c->snt * snapcell;
     } else {
         c->snap_stride = (size_t)c->keep * (c->S / c->g.snap_dt) * snapcell;   // >= one unit
-        for (int i = 0; i < 5; ++i) c->rf[i] = F(B * fs);
-        for (int i = 0; i < 4; ++i) c->rpsi[i] = F(B * c->psiz());
-        for (int i = 4; i < 8; ++i) c->rpsi[i] = F(B * c->psix());
-        if (c->fusable) level2(c->rf2, c->rpsi2);
-        c->ck_bytes_per_seg = sizeof(float) * B * (5 * fs + 4 * (c->psiz() + c->psix()));
+        for (int i = 0; i < 5; ++i) c->rf[i] = F(Bg * fs);
+        for (int i = 0; i < 4; ++i) c->rpsi[i] = F(Bg * c->psiz());
+        for (int i = 4; i < 8; ++i) c->rpsi[i] = F(Bg * c->psix());
+        if (c->fusable) level2(c->rf2, c->rpsi2, Bg);
+        c->ck_bytes_per_seg = sizeof(float) * Bg * (5 * fs + 4 * (c->psiz() + c->psix()));
         c->ck = F(c->ck_bytes_per_seg / sizeof(float) * std::max(c->slots, 1));
         c->rf_canon = c->rf[0];
     }
-    for (int i = 0; i < 5; ++i) c->snap[i] = F(B * c->snap_stride);
+    for (int i = 0; i < 5; ++i) c->snap[i] = F(Bg * c->snap_stride);
     if (c->o.seis_fp64) {
         c->d64 = D(15 * (size_t)B * fs);
         c->dmed = D(5 * fs);
@@ -1683,7 +1738,7 @@ int setup_device(fwi_ctx *c, const fwi_acq *q) {
     RETIF(allocate(c));
     // snapshot cells outside the interior are never written by the one-pass step: zero once
     for (int i = 0; i < 5; ++i)
-        HIPCHK(hipMemsetAsync(c->snap[i], 0, sizeof(float) * c->B * c->snap_stride, c->st));
+        HIPCHK(hipMemsetAsync(c->snap[i], 0, sizeof(float) * c->Bg * c->snap_stride, c->st));
     {   // per-step tables for graph replay (what time_step / adj_step derive from it)
         const int nt = c->g.nt, sdt = c->g.snap_dt;
         const long long slab = (long long)c->snz * c->snx;
@@ -2054,7 +2109,7 @@ int32_t fwi_forward(fwi_ctx *c, int32_t shot0, int32_t nshots, double *seis_z, d
     if (!c) return FWI_EINVAL;
     if (!c->have_model) return c->fail(FWI_ESTATE, "fwi_forward before fwi_set_model");
     std::vector<std::pair<int, int>> bs;
-    if (batches(c, shot0, nshots, bs) != FWI_OK) return c->fail(FWI_EINVAL, "shot range");
+    if (batches(c, shot0, nshots, c->B, bs) != FWI_OK) return c->fail(FWI_EINVAL, "shot range");
     const int nt = c->g.nt;
     for (auto [s0, nb] : bs) {
         RETIF(run_forward(c, s0, nb, false, !c->o.seis_fp64, true));
@@ -2076,7 +2131,7 @@ int32_t fwi_forward_device(fwi_ctx *c, int32_t shot0, int32_t nshots, double *se
     if (!c) return FWI_EINVAL;
     if (!c->have_model) return c->fail(FWI_ESTATE, "fwi_forward_device before a model");
     std::vector<std::pair<int, int>> bs;
-    if (batches(c, shot0, nshots, bs) != FWI_OK) return c->fail(FWI_EINVAL, "shot range");
+    if (batches(c, shot0, nshots, c->B, bs) != FWI_OK) return c->fail(FWI_EINVAL, "shot range");
     const int nt = c->g.nt;
     for (auto [s0, nb] : bs) {
         RETIF(run_forward(c, s0, nb, false, !c->o.seis_fp64, true));
@@ -2132,14 +2187,14 @@ int32_t fwi_gradient(fwi_ctx *c, int32_t shot0, int32_t nshots, double *misfit) 
     if (!c) return FWI_EINVAL;
     if (!c->have_model || !c->have_obs) return c->fail(FWI_ESTATE, "fwi_gradient needs a model and observed data");
     std::vector<std::pair<int, int>> bs;
-    if (batches(c, shot0, nshots, bs) != FWI_OK) return c->fail(FWI_EINVAL, "shot range");
+    if (batches(c, shot0, nshots, c->Bg, bs) != FWI_OK) return c->fail(FWI_EINVAL, "shot range");
     const int nz = c->g.nz, nx = c->g.nx;
     for (auto [s0, nb] : bs) {
         RETIF(batch_gradient(c, s0, nb, nullptr, nullptr, misfit ? misfit + (s0 - shot0) : nullptr));
         const size_t snapcell = (size_t)c->snz * c->snx;
         for (int s = 0; s < nb; ++s) {
             const double alpha = c->alpha[s0 + s];
-            const size_t cells = (size_t)c->B * snapcell;
+            const size_t cells = (size_t)c->Bg * snapcell;
             const double *gs[3] = {c->gr64 + s * snapcell, c->gr64 + cells + s * snapcell,
                                    c->gr64 + 2 * cells + s * snapcell};
             const double gsc[3] = {1.0 / (alpha * kGainLM), 1.0 / (alpha * kGainLM), 1.0 / alpha};
@@ -2157,19 +2212,19 @@ int32_t fwi_gradient_raw(fwi_ctx *c, int32_t shot0, int32_t nshots, const double
     if (!c || !adj_z || !adj_x) return FWI_EINVAL;
     if (!c->have_model) return c->fail(FWI_ESTATE, "fwi_gradient_raw before fwi_set_model");
     std::vector<std::pair<int, int>> bs;
-    if (batches(c, shot0, nshots, bs) != FWI_OK) return c->fail(FWI_EINVAL, "shot range");
+    if (batches(c, shot0, nshots, c->Bg, bs) != FWI_OK) return c->fail(FWI_EINVAL, "shot range");
     const size_t snapcell = (size_t)c->snz * c->snx;
     double *outs[3] = {g_lam, g_mu, g_rho};
     for (int k = 0; k < 3; ++k)
         if (outs[k]) std::memset(outs[k], 0, snapcell * 8);
-    std::vector<double> h(snapcell * c->B);
+    std::vector<double> h(snapcell * c->Bg);
     const int nt = c->g.nt, rb = c->rec_off[shot0];
     for (auto [s0, nb] : bs) {
         const size_t off = (size_t)(c->rec_off[s0] - rb) * nt;
         RETIF(batch_gradient(c, s0, nb, adj_z + off, adj_x + off, nullptr));
         for (int k = 0; k < 3; ++k) {
             if (!outs[k]) continue;
-            HIPCHK(hipMemcpyAsync(h.data(), c->gr64 + (size_t)k * c->B * snapcell, snapcell * nb * 8,
+            HIPCHK(hipMemcpyAsync(h.data(), c->gr64 + (size_t)k * c->Bg * snapcell, snapcell * nb * 8,
                                   hipMemcpyDeviceToHost, c->st));
             RETIF(sync(c));
             for (int s = 0; s < nb; ++s) {
@@ -2190,8 +2245,8 @@ int misfit_gradient_dev(fwi_ctx *c, int shot0, int nshots, const double *adj_z, 
     if (c->g.snap_dz != 1 || c->g.snap_dx != 1)
         return c->fail(FWI_EINVAL, "the misfit derivative needs snap_dz = snap_dx = 1 (staggered chain rule)");
     std::vector<std::pair<int, int>> bs;
-    if (batches(c, shot0, nshots, bs) != FWI_OK) return c->fail(FWI_EINVAL, "shot range");
-    const size_t snapcell = (size_t)c->snz * c->snx, cells = (size_t)c->B * snapcell;
+    if (batches(c, shot0, nshots, c->Bg, bs) != FWI_OK) return c->fail(FWI_EINVAL, "shot range");
+    const size_t snapcell = (size_t)c->snz * c->snx, cells = (size_t)c->Bg * snapcell;
     if (!c->raw) {   // FP64 totals of the five sums over the shots, allocated on first use
         c->raw = c->dalloc<double>(5 * snapcell);
         if (!c->raw) return c->fail(FWI_ENOMEM, "misfit-derivative sums");
@@ -2600,7 +2655,7 @@ int32_t fwi_misfit(fwi_ctx *c, int32_t shot0, int32_t nshots, double *L2) {
     if (!c || !L2) return FWI_EINVAL;
     if (!c->have_model || !c->have_obs) return c->fail(FWI_ESTATE, "fwi_misfit needs a model and observed data");
     std::vector<std::pair<int, int>> bs;
-    if (batches(c, shot0, nshots, bs) != FWI_OK) return c->fail(FWI_EINVAL, "shot range");
+    if (batches(c, shot0, nshots, c->B, bs) != FWI_OK) return c->fail(FWI_EINVAL, "shot range");
     double total = 0;
     std::vector<double> m(c->B);
     for (auto [s0, nb] : bs) {
