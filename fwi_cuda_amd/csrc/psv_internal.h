@@ -221,12 +221,16 @@ void x_media_chain(const XArgs &x, int nb, const double *mu, const double *rho, 
                    double *d_lam, double *d_mu, double *d_rho, hipStream_t st);
 
 // ---- the resident propagation: many time steps in one launch (psv_resident.h) -----------
-// A tiling: shots per launch, tile size, tiles per shot, cells per thread, block and LDS size.
+// A tiling: shots per launch, tile size, tiles per shot, cells per thread (0: the kernel of
+// one exchange per step), block and LDS size.
 struct ResPlan {
     int shots, TX, TZ, ntx, ntz, cpt, threads;
     int psi_lds, psi_rows, psi_cols;   // CPML memory in LDS: a tile's strip rows and columns, at most
     size_t lds;
 };
+constexpr int kResItems = 4;    // edge values a thread reads per half-step, at most
+constexpr int kRes1Cells = 2;   // cells whose velocities a thread reads per step, at most (cpt 0)
+constexpr uint32_t res1_words(int TX, int TZ, int wpv) { return (uint32_t)(TX * TZ * 2 * wpv + 15) / 16u * 16u; }
 constexpr size_t kResLds = 160 * 1024;   // LDS of a CU
 // columns of a block's lanes (a tile is at most that wide) for a number of cells per thread
 constexpr int res_lanes(int cpt, int elt) { return cpt >= 4 && elt == 4 ? 64 : 32; }

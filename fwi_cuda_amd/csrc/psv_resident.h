@@ -37,7 +37,6 @@ namespace psv {
 namespace {
 
 constexpr int kSpinLimit = 1 << 22;
-constexpr int kResItems = 4;   // edge values a thread reads per half-step, at most
 
 template <class T>
 __device__ __forceinline__ void mail_put(unsigned long long *w, T v, uint32_t tag) {
@@ -712,10 +711,387 @@ __global__ __launch_bounds__(1024) void k_resident(const ResArgs<T> r) {
     }
 }
 
+// One exchange per step, for small tiles.  A thread owns one cell of the tile or of the N
+// cells around it and advances the stresses there too (the same operations on the same
+// values as their owner, so the same bits); only velocities travel, 2N cells deep.  A step
+// then waits once instead of twice, for N more rows and columns of stress arithmetic each
+// side and more words: worth it where a CU has threads to spare (at most 32 - 2N rows and
+// columns per tile).  A tile's words are its own lines of memory, two sets taken in turn: a block
+// overwrites the words of step n in step n + 2, after it has seen every neighbour's words
+// of step n + 1, which they write after the barrier that follows their reads of step n.
+// Measured per forward step against two exchanges: 72 x 96, 3 shots 4.1 -> 3.2 us, 201 x 401
+// 4.1 -> 3.7; forward and adjoint step 201 x 401 8.7 -> 7.5.  The FP64 propagation's words
+// are twice as many: 10.1 -> 11.1, so it keeps the two exchanges.  A tile's words lie
+// together: at their cell's place in one array (lines written by several blocks) 17 x 15
+// tiles took 4.4 instead of 3.9; rows of 32 lanes: packed to the tile's width they take
+// fewer wavefronts but 4.0 instead of 3.7.
+template <class T, int N, bool ADJ>
+__global__ __launch_bounds__(1024) void k_resident1(const ResArgs<T> r) {
+    extern __shared__ char smem[];
+    constexpr int WPV = (int)sizeof(T) / 4;
+    constexpr int VA = 32 + 2 * N, VW = 2 * VA, SA = 32, SW = 3 * SA;
+    const int t = threadIdx.x, nthr = blockDim.x;
+    const int TX = r.TX, TZ = r.TZ;
+    T *lvz = reinterpret_cast<T *>(smem), *lvx = lvz + VA;                 // [TZ + 4N][2][VA]
+    T *lzz = lvz + (TZ + 4 * N) * VW, *lzx = lzz + SA, *lxx = lzx + SA;    // [TZ + 2N][3][SA]
+    T *zprof = lzz + (TZ + 2 * N) * SW;                                    // [TZ + 2N][6]
+    const int blk = blockIdx.x, tx = blk % r.ntx, ty = blk / r.ntx % r.ntz, ls = blk / (r.ntx * r.ntz);
+    const int s = r.s0 + ls;
+    const int x0 = N + tx * TX, z0 = N + ty * TZ;
+    const int w = min(TX, r.nx - N - x0), h = min(TZ, r.nz - N - z0);
+    const int lx = t % 32, lz = t / 32;                    // cell (x0 - N + lx, z0 - N + lz)
+    const int ix = x0 - N + lx, iz = z0 - N + lz;
+    const bool own = lx >= N && lx < N + w && lz >= N && lz < N + h;
+    const bool ext = lx < w + 2 * N && lz < h + 2 * N && ix >= N && ix < r.nx - N && iz >= N && iz < r.nz - N;
+    const size_t P = r.P, fo = (size_t)s * r.fs;
+    const size_t m = ext ? (size_t)iz * P + ix : 0;
+    const T dt = r.dt;
+
+    int *cellmap = reinterpret_cast<int *>(smem);
+    for (int i = t; i < 32 * (TZ + 2 * N); i += nthr) cellmap[i] = 0;
+    __syncthreads();
+    for (int k = 0; k < 2; ++k) {
+        const SrcArgs &a = k ? r.rec : r.src;
+        for (int g = t; g < a.ngroups; g += nthr) {
+            const int cell = a.grp_cell[g], cz = cell / r.P - z0, cx = cell % r.P - x0;
+            if (a.grp_shot[g] - r.shot0 == s && cz >= 0 && cz < h && cx >= 0 && cx < w)
+                cellmap[(cz + N) * 32 + cx + N] |= (g + 1) << (16 * k);
+        }
+        __syncthreads();
+    }
+    const int pt = own ? cellmap[lz * 32 + lx] : 0;
+    const int gsrc = (pt & 0xffff) - 1, grec = (int)((unsigned)pt >> 16) - 1;
+    __syncthreads();
+
+    for (int j = t; j < (TZ + 4 * N) * VA; j += nthr) {
+        const int cz = z0 - 2 * N + j / VA, cx = x0 - 2 * N + j % VA, i = j / VA * VW + j % VA;
+        const bool in = r.load && cz >= 0 && cz < r.nz && cx >= 0 && cx < r.nx;
+        const size_t o = fo + (size_t)cz * P + cx;
+        lvz[i] = in ? r.vz[o] : T(0);
+        lvx[i] = in ? r.vx[o] : T(0);
+    }
+    for (int j = t; j < (TZ + 2 * N) * SW; j += nthr) lzz[j] = T(0);
+    for (int i = t; i < TZ + 2 * N; i += nthr) {
+        const int cz = min(max(z0 - N + i, 0), r.nz - 1);
+        const CpmlPoint p = r.zp[cz];
+        for (int k = 0; k < 6; ++k) zprof[i * 6 + k] = prof_at(r, p, r.zpf, cz, k);
+    }
+    const CpmlPoint xpt = r.xp[ext ? ix : N];
+    const int cxp = ext ? ix : N;
+    const int xm = ext ? xpt.map : -1, zm = ext ? r.zp[iz].map : -1;
+    const T xb = prof_at(r, xpt, r.xpf, cxp, 0), xa = prof_at(r, xpt, r.xpf, cxp, 1), xk = prof_at(r, xpt, r.xpf, cxp, 2),
+            xbh = prof_at(r, xpt, r.xpf, cxp, 3), xah = prof_at(r, xpt, r.xpf, cxp, 4),
+            xkh = prof_at(r, xpt, r.xpf, cxp, 5);
+    const T lam = ext ? r.lam[m] : T(0), mu = ext ? r.mu[m] : T(0), muzx = ext ? r.muzx[m] : T(0);
+    const T rhoz = own ? r.rhoz[m] : T(0), rhox = own ? r.rhox[m] : T(0);
+    const bool ld = r.load && ext;
+    T szz = ld ? r.szz[fo + m] : T(0), szx = ld ? r.szx[fo + m] : T(0), sxx = ld ? r.sxx[fo + m] : T(0);
+    T vz = ld && own ? r.vz[fo + m] : T(0), vx = ld && own ? r.vx[fo + m] : T(0);
+    T we = own && r.energy ? r.We[fo + m] : T(0), uz = T(0), ux = T(0);
+    if constexpr (ADJ) {
+        if (own) uz = r.uz[fo + m], ux = r.ux[fo + m];
+    }
+    auto psi_at = [&](RSeg<T> q, int j) -> T * {
+        return j < 4 ? q->psi[j] + ((size_t)s * q->nzs + zm) * q->P + ix
+                     : q->psi[j] + ((size_t)s * q->nz + iz) * q->nxs + xm;
+    };
+    // the stress pass's memories (slots 0, 1, 4, 5) belong to every cell the thread advances,
+    // the velocity pass's to its own
+    auto psi_in = [&](int j) { return (j < 4 ? zm >= 0 : xm >= 0) && ((j & 2) == 0 || own); };
+    T pr[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) pr[j] = r.load && psi_in(j) ? *psi_at(res_seg<T>(), j) : T(0);
+    const bool zs = zm >= 0, xs = xm >= 0, top_row = ext && iz == r.surf;
+
+    const bool lat = own && ix >= r.snap_x1 && ix <= r.snap_x2 && (ix - r.snap_x1) % r.snap_dx == 0 &&
+                     iz >= r.snap_z1 && iz <= r.snap_z2 && (iz - r.snap_z1) % r.snap_dz == 0;
+    const uint32_t lc = lat ? (uint32_t)((iz - r.snap_z1) / r.snap_dz * r.snx + (ix - r.snap_x1) / r.snap_dx) : 0u;
+    const size_t slab = (size_t)r.snz * r.snx;
+    const int ng = ADJ ? (r.gform ? 5 : 3) : 0;
+    T gs[ADJ ? 5 : 1];
+    if constexpr (ADJ) {
+#pragma unroll
+        for (int j = 0; j < 5; ++j) gs[j] = j < ng && lat ? r.g[j][(size_t)s * slab + lc] : T(0);
+    }
+
+    // the words this thread reads: velocities of the cells within 2N of the tile
+    const uint32_t tw = res1_words(TX, TZ, WPV), set = gridDim.x * tw;   // words of a tile, of a set
+    auto word = [&](int cz, int cx) {           // of the cell's owner
+        const int ox = (cx - N) / TX, oz = (cz - N) / TZ;
+        return (uint32_t)((ls * r.ntz + oz) * r.ntx + ox) * tw +
+               (uint32_t)((cz - N - oz * TZ) * TX + cx - N - ox * TX) * 2u * WPV;
+    };
+    uint32_t mw[kRes1Cells];
+    int ml[kRes1Cells];
+    int nit = 0;
+#pragma unroll
+    for (int q = 0; q < kRes1Cells; ++q) {
+        mw[q] = 0;
+        ml[q] = -1;
+        const int i = t + q * nthr;
+        if (i >= (w + 4 * N) * (h + 4 * N)) continue;
+        const int rx = i % (w + 4 * N), rz = i / (w + 4 * N), cx = x0 - 2 * N + rx, cz = z0 - 2 * N + rz;
+        if (cx < N || cx >= r.nx - N || cz < N || cz >= r.nz - N) continue;
+        if (rx >= 2 * N && rx < 2 * N + w && rz >= 2 * N && rz < 2 * N + h) continue;
+        mw[q] = word(cz, cx);
+        ml[q] = rz * VW + rx;
+        nit = q + 1;
+    }
+    const bool alone = r.ntx * r.ntz == 1;
+    const uint32_t mine = own ? word(iz, ix) : 0u;
+    bool dead = false;
+    auto receive = [&](uint32_t tag, int parity) {
+        const RSeg<T> sg = res_seg<T>();
+        const unsigned long long *base = sg->mail + (parity ? set : 0u);
+        unsigned long long v[kRes1Cells][2 * WPV];
+#pragma unroll
+        for (int q = 0; q < kRes1Cells; ++q)
+            if (ml[q] >= 0)
+#pragma unroll
+                for (int j = 0; j < 2 * WPV; ++j) v[q][j] = mail_get(base + mw[q] + j);
+#pragma unroll
+        for (int q = 0; q < kRes1Cells; ++q)
+            if (ml[q] >= 0) {
+#pragma unroll
+                for (int j = 0; j < 2 * WPV; ++j) {
+                    int spin = 0;
+                    while ((uint32_t)(v[q][j] >> 32) != tag && !dead) {
+                        v[q][j] = mail_get(base + mw[q] + j);
+                        if (++spin > kSpinLimit) {
+                            dead = true;
+                            __hip_atomic_store(sg->err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                        }
+                    }
+                }
+#pragma unroll
+                for (int f = 0; f < 2; ++f) {
+                    T val;
+                    if constexpr (sizeof(T) == 4)
+                        val = __uint_as_float((uint32_t)v[q][f]);
+                    else
+                        val = __longlong_as_double((long long)((v[q][2 * f] & 0xffffffffull) | v[q][2 * f + WPV - 1] << 32));
+                    lvz[ml[q] + f * VA] = val;
+                }
+            }
+    };
+    auto source_row = [&](int j, int it, T &dz, T &dx) {
+        const RSeg<T> q = res_seg<T>();
+        const auto &a = q->src;
+        const size_t row = (size_t)a.grp_idx[j] * a.nt + it;
+        const double sc = a.scale_shot ? a.scale_shot[q->shot0 + s] : 1.0;
+        const double fz = a.stf_z[row] * sc, fx = a.stf_x[row] * sc;
+        if (a.type == 0) {
+            dz = (T)(a.dt * (double)rhoz * fz / a.dzdx);
+            dx = (T)(a.dt * (double)rhox * fx / a.dzdx);
+        } else {
+            dz = (T)fz;
+            dx = (T)fx;
+        }
+    };
+    __syncthreads();
+
+    const int vc = (lz + N) * VW + lx + N, sc_ = lz * SW + lx;   // the cell in the two LDS planes
+    for (int n = 0; n < r.nsteps; ++n) {
+        const int it = r.t0 + r.dir * n;
+        const uint32_t tag = r.epoch + (uint32_t)n;
+        int c = vc, d = sc_;
+        asm volatile("" : "+v"(c), "+v"(d));
+        T pdz = T(0), pdx = T(0);               // the first source's increments, read ahead of the wait
+        if (gsrc >= 0) source_row(res_seg<T>()->src.grp_off[gsrc], it, pdz, pdx);
+        const bool gstep = ADJ && it % r.snap_dt == 0;
+        T S[ADJ ? 5 : 1];
+        if constexpr (ADJ) {
+            if (gstep && lat) {                 // what a correlating step reads, too
+                const RSeg<T> q = res_seg<T>();
+                const size_t o = (size_t)s * q->sn_stride + (size_t)((it - q->tb) / q->snap_dt) * slab + lc;
+#pragma unroll
+                for (int j = 0; j < 5; ++j) S[j] = q->sn[j][o];
+            }
+        }
+        if (n > 0 && nit) receive(tag - 1u, (n - 1) & 1);
+        lds_barrier();
+        if (ext) {                              // ---- stress half-step
+            T vz_z = 0, vx_z = 0, vz_x = 0, vx_x = 0;
+#pragma unroll
+            for (int i = 1; i <= N; ++i) {
+                vz_z += r.cz[i - 1] * (lvz[c + (i - 1) * VW] - lvz[c - i * VW]);
+                vx_z += r.cz[i - 1] * (lvx[c + i * VW] - lvx[c - (i - 1) * VW]);
+                vz_x += r.cx[i - 1] * (lvz[c + i] - lvz[c + 1 - i]);
+                vx_x += r.cx[i - 1] * (lvx[c + i - 1] - lvx[c - i]);
+            }
+            if (zs) {
+                const T *pf = zprof + lz * 6;
+                const T p1 = pf[0] * pr[0] + pf[1] * vz_z, p2 = pf[3] * pr[1] + pf[4] * vx_z;
+                pr[0] = p1;
+                pr[1] = p2;
+                vz_z = vz_z * pf[2] + p1;
+                vx_z = vx_z * pf[5] + p2;
+            }
+            if (xs) {
+                const T p1 = xb * pr[4] + xa * vx_x, p2 = xbh * pr[5] + xah * vz_x;
+                pr[4] = p1;
+                pr[5] = p2;
+                vx_x = vx_x * xk + p1;
+                vz_x = vz_x * xkh + p2;
+            }
+            if constexpr (!ADJ && sizeof(T) == 4) {
+                if (r.hist && own) {
+                    T *hp = res_seg<T>()->hist + ((size_t)(it - r.hist_base) * r.hist_B + s) * 5 * r.fs + m;
+                    hp[0] = vz_z;
+                    hp[r.fs] = vx_x;
+                    hp[2 * r.fs] = vz_x + vx_z;
+                }
+            }
+            const T div = lam * (vx_x + vz_z);
+            szz = szz + dt * (div + T(2) * mu * vz_z);
+            szx = szx + dt * muzx * (vz_x + vx_z);
+            sxx = sxx + dt * (div + T(2) * mu * vx_x);
+            if (top_row) {                      // surf_mirror at row N (src/cpu/n_kernel_lib_PSV.cpp:297-301)
+                szz = 0;
+                szx = 0;
+                sxx = T(4) * dt * vx_x * (lam * mu + mu * mu) / (lam + T(2) * mu);
+            }
+            lzz[d] = szz;
+            lzx[d] = szx;
+            lxx[d] = sxx;
+        }
+        lds_barrier();
+        if (own) {                              // ---- velocity half-step
+            T szz_z = 0, szx_z = 0, szx_x = 0, sxx_x = 0;
+#pragma unroll
+            for (int i = 1; i <= N; ++i) {
+                szz_z += r.cz[i - 1] * (lzz[d + i * SW] - lzz[d - (i - 1) * SW]);
+                szx_z += r.cz[i - 1] * (lzx[d + (i - 1) * SW] - lzx[d - i * SW]);
+                szx_x += r.cx[i - 1] * (lzx[d + i - 1] - lzx[d - i]);
+                sxx_x += r.cx[i - 1] * (lxx[d + i] - lxx[d + 1 - i]);
+            }
+            if (zs) {
+                const T *pf = zprof + lz * 6;
+                const T p1 = pf[0] * pr[2] + pf[1] * szz_z, p2 = pf[3] * pr[3] + pf[4] * szx_z;
+                pr[2] = p1;
+                pr[3] = p2;
+                szz_z = szz_z * pf[2] + p1;
+                szx_z = szx_z * pf[5] + p2;
+            }
+            if (xs) {
+                const T p1 = xb * pr[6] + xa * sxx_x, p2 = xbh * pr[7] + xah * szx_x;
+                pr[6] = p1;
+                pr[7] = p2;
+                sxx_x = sxx_x * xk + p1;
+                szx_x = szx_x * xkh + p2;
+            }
+            if constexpr (!ADJ && sizeof(T) == 4) {
+                if (r.hist) {
+                    T *hp = res_seg<T>()->hist + (((size_t)(it - r.hist_base) * r.hist_B + s) * 5 + 3) * r.fs + m;
+                    hp[0] = szx_x + szz_z;
+                    hp[r.fs] = sxx_x + szx_z;
+                }
+            }
+            const T vz0 = vz, vx0 = vx;
+            T vz1 = vz0 + dt * rhoz * (szx_x + szz_z);
+            T vx1 = vx0 + dt * rhox * (sxx_x + szx_z);
+            if constexpr (ADJ) {
+                uz = uz + dt * vz0;
+                ux = ux + dt * vx0;
+            }
+            if (r.energy) we = we + (vx1 * vx1 + vz1 * vz1);
+            const T pvz = vz1, pvx = vx1;       // before the injection
+            if (gsrc >= 0) {                    // vsrc2: the group's sources in source order
+                const RSeg<T> q = res_seg<T>();
+                vz1 += pdz;
+                vx1 += pdx;
+                for (int j = q->src.grp_off[gsrc] + 1; j < q->src.grp_off[gsrc + 1]; ++j) {
+                    T dz, dx;
+                    source_row(j, it, dz, dx);
+                    vz1 += dz;
+                    vx1 += dx;
+                }
+            }
+            vz = vz1;
+            vx = vx1;
+            lvz[c] = vz1;
+            lvx[c] = vx1;
+            if (!alone && n + 1 < r.nsteps) {
+                unsigned long long *o = res_seg<T>()->mail + (n & 1 ? set : 0u) + mine;
+                mail_put(o, vz1, tag);
+                mail_put(o + WPV, vx1, tag);
+            }
+            if (grec >= 0) {                    // the velocity sample; k_seis_scan makes urec2's running sum
+                const RSeg<T> q = res_seg<T>();
+                for (int j = q->rec.grp_off[grec]; j < q->rec.grp_off[grec + 1]; ++j) {
+                    const size_t o = (size_t)q->rec.grp_idx[j] * q->rec.nt + it;
+                    q->seis_z[o] = (double)vz1;
+                    q->seis_x[o] = (double)vx1;
+                }
+            }
+            if constexpr (ADJ) {
+                if (lat) {
+                    if (gstep) {                // fwi_grad2 (:439-484)
+                        const T Vz = S[0], Vx = S[1], Szz = S[2], Szx = S[3], Sxx = S[4];
+                        const T lm = lam + mu;
+                        const T il = r.gain_lm / (lm * lm), im = r.gain_lm / (mu * mu);
+                        const T s1 = T(0.25) * il * (Szz + Sxx) * (szz + sxx);
+                        const T s2 = T(0.25) * im * (Szz - Sxx) * (szz - sxx);
+                        const T s3 = im * (Szx * szx);
+                        gs[0] = gs[0] + r.gw * s1;
+                        if (!r.gform) {
+                            gs[1] = gs[1] + r.gw * (s3 + s1 + s2);
+                            gs[2] = gs[2] + r.gw * (ux * Vx + uz * Vz);
+                        } else {
+                            gs[1] = gs[1] + r.gw * (s1 + s2);
+                            gs[2] = gs[2] + r.gw * (dt * (pvz * Vz));
+                            gs[3] = gs[3] + r.gw * s3;
+                            gs[4] = gs[4] + r.gw * (dt * (pvx * Vx));
+                        }
+                    }
+                    if ((r.nt - it) % r.flush_every == 0) {   // the FP32 sums into their FP64 totals
+                        const RSeg<T> q = res_seg<T>();
+#pragma unroll
+                        for (int j = 0; j < 5; ++j)
+                            if (j < ng) {
+                                q->g64[j * q->g64_stride + (size_t)s * slab + lc] += (double)gs[j];
+                                gs[j] = T(0);
+                            }
+                    }
+                }
+            } else {
+                if (r.store && lat && it >= r.tb && it % r.snap_dt == 0) {   // gard_fwd_storage2
+                    const RSeg<T> q = res_seg<T>();
+                    const size_t o = (size_t)s * q->st_stride + (size_t)((it - q->tb) / q->snap_dt) * slab + lc;
+                    q->st[0][o] = vz1 / dt;
+                    q->st[1][o] = vx1 / dt;
+                    q->st[2][o] = szz;
+                    q->st[3][o] = szx;
+                    q->st[4][o] = sxx;
+                }
+            }
+        }
+    }
+
+    if (!r.load || !own) return;
+    r.vz[fo + m] = vz;
+    r.vx[fo + m] = vx;
+    r.szz[fo + m] = szz;
+    r.szx[fo + m] = szx;
+    r.sxx[fo + m] = sxx;
+    if (r.energy) r.We[fo + m] = we;
+    if constexpr (ADJ) {
+        r.uz[fo + m] = uz;
+        r.ux[fo + m] = ux;
+#pragma unroll
+        for (int j = 0; j < 5; ++j)
+            if (j < ng && lat) r.g[j][(size_t)s * slab + lc] = gs[j];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+        if (psi_in(j)) *psi_at(res_seg<T>(), j) = pr[j];
+}
+
 template <class T, bool ADJ, int N>
 hipError_t launch_resident_n(const ResArgs<T> &r, int cpt, int blocks, int threads, size_t lds, hipStream_t st) {
     constexpr int E = (int)sizeof(T);
-    const void *f = cpt == 1   ? (const void *)k_resident<T, N, 1, res_lanes(1, E), ADJ>
+    const void *f = cpt == 0   ? (const void *)k_resident1<T, N, ADJ>
+                    : cpt == 1 ? (const void *)k_resident<T, N, 1, res_lanes(1, E), ADJ>
                     : cpt == 2 ? (const void *)k_resident<T, N, 2, res_lanes(2, E), ADJ>
                     : cpt == 4 ? (const void *)k_resident<T, N, 4, res_lanes(4, E), ADJ>
                                : (const void *)k_resident<T, N, E == 8 ? 4 : 8, res_lanes(E == 8 ? 4 : 8, E), ADJ>;

@@ -55,7 +55,7 @@ int strip_lines(const std::vector<int> &map, int N, int T) {
 // their registers and words do; that sweep with four cells per thread spills its FP64 sums
 // (301 x 601, 4 shots: 31 us a step against 2 x 10 for two launches of two cells per
 // thread).  Every tile holds at least N rows and columns (its halo comes from direct
-// neighbours only).  FP32 steps that the batched kernels run as fast, at 16 us of launches
+// neighbours only; the one-exchange kernel, 0 cells per thread, has none such).  FP32 steps that the batched kernels run as fast, at 16 us of launches
 // and 14.4 us per million cells, are left to them: 600 x 1100, 8 shots take 78 us there and
 // 82 here, 800 x 1400, 1 shot 35 and 26.
 bool plan_resident(int nz, int nx, int N, int nb, ResUse use, int cus, size_t lds, const std::vector<int> &zmap,
@@ -72,7 +72,24 @@ bool plan_resident(int nz, int nx, int N, int nb, ResUse use, int cus, size_t ld
             const int TX = (ix + ntx - 1) / ntx;
             if (TX > 64 || (ntx > 1 && ix - (ntx - 1) * TX < N)) continue;
             const int cols = strip_lines(xmap, N, TX);
-            for (int ntz = 1; ntz <= std::min(tiles / ntx, iz); ++ntz)
+            for (int ntz = 1; ntz <= std::min(tiles / ntx, iz); ++ntz) {
+                // one exchange per step; tiles that fill the 32 lanes measured 5 % slower than the
+                // next narrower ones (201 x 401: 24 x 13 cells 3.9 us, 22 x 14 3.7, 16 x 20 3.7)
+                if (use != kUseExact && use != kUseFp64 && TX + 2 * N < 32) {
+                    const int TZ = (iz + ntz - 1) / ntz;
+                    const int thr = (32 * (TZ + 2 * N) + 63) / 64 * 64;
+                    if (thr <= 1024 && iz - (ntz - 1) * TZ > 0 &&
+                        (TX + 4 * N) * (TZ + 4 * N) <= kRes1Cells * thr) {
+                        // tiles narrower than the frame wait for their neighbours' neighbours too
+                        const bool thin = (ntx > 1 && TX < 2 * N) || (ntz > 1 && TZ < 2 * N);
+                        const double t = launches * (2.3 - (ntx * ntz == 1 ? 1.2 : 0.0) + (thin ? 0.5 : 0.0) + 1.1e-3 * thr);
+                        if (t < best) {
+                            best = t;
+                            *out = {g, TX, TZ, ntx, ntz, 0, thr, 0, 0, 0,
+                                    (size_t)elt * (2 * (32 + 2 * N) * (TZ + 4 * N) + (3 * 32 + 6) * (TZ + 2 * N))};
+                        }
+                    }
+                }
                 for (int cpt : {1, 2, 4, 8}) {
                     if (cpt > max_cpt || TX > res_lanes(cpt, elt)) continue;
                     const int rows = (iz + ntz - 1) / ntz, TZ = (rows + cpt - 1) / cpt * cpt;
@@ -97,6 +114,7 @@ bool plan_resident(int nz, int nx, int N, int nb, ResUse use, int cus, size_t ld
                         *out = {g, TX, TZ, ntx, ntz, cpt, thr, psi_lds, srows, cols, need};
                     }
                 }
+            }
         }
     }
     return best < (use == kUseStep ? 0.9 * (16.0 + 14.4e-6 * nb * nz * nx) : 1e299);
@@ -119,6 +137,7 @@ void launch_seis_scan(double *z, double *x, int rows, int nt, double dt, double 
 }
 
 size_t resident_words(const ResPlan &p, int N, int elt) {
+    if (p.cpt == 0) return (size_t)2 * p.shots * p.ntx * p.ntz * res1_words(p.TX, p.TZ, elt / 4);
     return (size_t)2 * p.shots * p.ntx * p.ntz * 4 * N * (p.TX + p.TZ) * (elt / 4);
 }
 
