@@ -152,6 +152,7 @@ struct fwi_ctx {
 
     // ---- the resident propagation (psv_resident.h): tilings per batch size
     // (shots 0: none), edge words, the next launch's first tag, flag of a wait that gave up
+    // (device memory, beside nonfinite)
     bool res_grid = false;   // the grid, acquisition and device allow it
     int cus = 0;
     std::vector<int> zmap_h, xmap_h;
@@ -159,7 +160,7 @@ struct fwi_ctx {
     unsigned long long *mail = nullptr;
     size_t mail_words = 0;
     uint32_t mail_tag = 1;
-    int *res_err = nullptr;  // pinned host memory
+    int *res_err = nullptr;
     char *xws = nullptr;     // the exact adjoint's workspace, kept while it is small (kExactKeep)
     size_t xws_bytes = 0;
 
@@ -276,11 +277,17 @@ int sync(fwi_ctx *c) {
     e = hipGetLastError();
     if (e != hipSuccess) return c->fail(FWI_EHIP, "launch: %s", hipGetErrorString(e));
     prof_collect(c);
-    if (c->res_err && *(volatile int *)c->res_err) {
-        *c->res_err = 0;
-        return c->fail(FWI_EHIP, "resident propagation: a tile's neighbour did not answer");
-    }
     return FWI_OK;
+}
+
+// after resident launches: a wait that gave up (none does while every block is resident)
+int check_resident(fwi_ctx *c) {
+    int h = 0;
+    HIPCHK(hipMemcpyAsync(&h, c->res_err, sizeof(int), hipMemcpyDeviceToHost, c->st));
+    RETIF(sync(c));
+    if (!h) return FWI_OK;
+    HIPCHK(hipMemsetAsync(c->res_err, 0, sizeof(int), c->st));
+    return c->fail(FWI_EHIP, "resident propagation: a tile's neighbour did not answer");
 }
 
 template <class T>
@@ -737,14 +744,15 @@ int ckpt_copy(fwi_ctx *c, int k, int nb, const Wave &w, bool save) {
 }
 
 int check_finite(fwi_ctx *c, int nb) {
-    if (!c->o.check_finite) return FWI_OK;
+    if (!c->o.check_finite) return resident(c, nb) ? check_resident(c) : FWI_OK;
     HIPCHK(hipMemsetAsync(c->nonfinite, 0, sizeof(int), c->st));
     dev_count_nonfinite(c->f[0], nb * c->fs(), c->nonfinite, c->st);
     dev_count_nonfinite(c->f[1], nb * c->fs(), c->nonfinite, c->st);
-    int h = 0;
-    HIPCHK(hipMemcpyAsync(&h, c->nonfinite, sizeof(int), hipMemcpyDeviceToHost, c->st));
+    int h[2] = {0, 0};   // and the resident propagation's flag
+    HIPCHK(hipMemcpyAsync(h, c->nonfinite, 2 * sizeof(int), hipMemcpyDeviceToHost, c->st));
     RETIF(sync(c));
-    if (h) return c->fail(FWI_ENONFINITE, "%d non-finite velocity values after propagation", h);
+    if (h[1]) return check_resident(c);
+    if (h[0]) return c->fail(FWI_ENONFINITE, "%d non-finite velocity values after propagation", h[0]);
     return FWI_OK;
 }
 
@@ -1287,7 +1295,7 @@ int run_forward64(fwi_ctx *c, int s0, int nb) {
             HIPCHK(launch_resident_fp64(r, *p, c->N, ns, c->st));
         }
         resident_seismograms(c, s0, nb);
-        return FWI_OK;
+        return check_resident(c);
     }
     int isurf[4];
     for (int k = 0; k < 4; ++k) isurf[k] = c->g.isurf[k];
@@ -1592,7 +1600,8 @@ int allocate(fwi_ctx *c) {
     c->tmp = D(2 * nn);
     c->red = D(4 + 3 * 1024);
     if (c->o.param == FWI_PARAM_VELOCITY) c->vel = D(4 * nn);
-    c->nonfinite = I(1);
+    c->nonfinite = I(2);
+    c->res_err = c->nonfinite ? c->nonfinite + 1 : nullptr;
     c->zmap = I(nz);
     c->xmap = I(nx);
     for (int i = 0; i < 6; ++i) c->pf[i] = F(nz);
@@ -1729,13 +1738,10 @@ int setup_device(fwi_ctx *c, const fwi_acq *q) {
         c->zmap_h = zmap;
         c->xmap_h = xmap;
         c->res_grid = c->fusable && c->nsrc_tot < 32767 && c->nrec_tot < 32767 && cooperative_ok(c->o.device, c->st);
-        if (c->res_grid) {
-            HIPCHK(hipHostMalloc((void **)&c->res_err, sizeof(int), hipHostMallocDefault));
-            *c->res_err = 0;
-        }
     }
     RETIF(plan(c));
     RETIF(allocate(c));
+    HIPCHK(hipMemsetAsync(c->res_err, 0, sizeof(int), c->st));
     // snapshot cells outside the interior are never written by the one-pass step: zero once
     for (int i = 0; i < 5; ++i)
         HIPCHK(hipMemsetAsync(c->snap[i], 0, sizeof(float) * c->Bg * c->snap_stride, c->st));
@@ -2017,7 +2023,6 @@ void fwi_destroy(fwi_ctx *c) {
     for (auto e : c->ev_pool) hipEventDestroy(e);
     free_all(c);
     if (c->xws) hipFree(c->xws);
-    if (c->res_err) hipHostFree(c->res_err);
     if (c->st) hipStreamDestroy(c->st);
     delete c;
 }
@@ -2525,7 +2530,7 @@ int exact_gradient(fwi_ctx *c, int shot0, int nshots, const double *adj_z, const
         x.G = G;
         x_media_chain(x, nshots, c->m_mu, c->m_rho, c->g.snap_z1, c->g.snap_z2, c->g.snap_x1, c->g.snap_x2, d_lam,
                       d_mu, d_rho, c->st);
-        r = sync(c);
+        r = res ? check_resident(c) : sync(c);
     }
     release();
     return r;

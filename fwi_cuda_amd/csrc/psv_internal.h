@@ -267,7 +267,7 @@ struct ResArgs {
     double *seis_z, *seis_x;            // velocity samples, absolute rows [nt]
     unsigned long long *mail;           // edge words, resident_words() of them
     uint32_t epoch;                     // tag of the launch's first step
-    int *err;                           // host-visible: set when a wait gave up
+    int *err;                           // set when a wait gave up
 };
 // What a tiling is for: FP32 steps, the FP64 propagation, the exact adjoint's two passes.
 enum ResUse { kUseStep, kUseFp64, kUseExactForward, kUseExact };

@@ -1,6 +1,7 @@
 // psv_resident.hip -- the resident propagation (psv_resident.h): forward kernels, the tile
 // choice and the receivers' running sums.
 #include <algorithm>
+#include <atomic>
 
 #include "psv_resident.h"
 
@@ -122,13 +123,18 @@ bool plan_resident(int nz, int nx, int N, int nb, ResUse use, int cus, size_t ld
 
 // Cooperative launches work: the attribute, and one empty launch (the runtime's cooperative
 // queue can be taken by another process of the same GPU; the steps then go launch by launch).
+// Once made, a process's queue stays, so a device that took the launch is not asked again.
 bool cooperative_ok(int device, hipStream_t st) {
+    static std::atomic<unsigned long long> known{0};
+    const unsigned long long bit = 1ull << (device & 63);
+    if (device < 64 && (known.load() & bit)) return true;
     int a = 0;
     if (hipDeviceGetAttribute(&a, hipDeviceAttributeCooperativeLaunch, device) != hipSuccess || !a) return false;
     if (hipLaunchCooperativeKernel((const void *)k_probe, dim3(1), dim3(64), nullptr, 0, st) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
+    if (device < 64) known.fetch_or(bit);
     return true;
 }
 
