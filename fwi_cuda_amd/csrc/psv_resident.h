@@ -719,6 +719,11 @@ __global__ __launch_bounds__(1024) void k_resident(const ResArgs<T> r) {
 // columns per tile).  A tile's words are its own lines of memory, two sets taken in turn: a block
 // overwrites the words of step n in step n + 2, after it has seen every neighbour's words
 // of step n + 1, which they write after the barrier that follows their reads of step n.
+// The rim is loaded from arrays that its owners overwrite when they end: a block stores its
+// state only after it has seen a word of every neighbour, which they write after their
+// loads.  From two steps on the exchange sees to that; a launch of one step makes the
+// exchange for that alone (k_resident waits for stress words in every step, and the exact
+// adjoint's sweep loads own cells only).
 // Measured per forward step against two exchanges: 72 x 96, 3 shots 4.1 -> 3.2 us, 201 x 401
 // 4.1 -> 3.7; forward and adjoint step 201 x 401 8.7 -> 7.5.  The FP64 propagation's words
 // are twice as many: 10.1 -> 11.1, so it keeps the two exchanges.  A tile's words lie
@@ -1011,7 +1016,7 @@ __global__ __launch_bounds__(1024) void k_resident1(const ResArgs<T> r) {
             vx = vx1;
             lvz[c] = vz1;
             lvx[c] = vx1;
-            if (!alone && n + 1 < r.nsteps) {
+            if (!alone && (n + 1 < r.nsteps || n == 0)) {
                 unsigned long long *o = res_seg<T>()->mail + (n & 1 ? set : 0u) + mine;
                 mail_put(o, vz1, tag);
                 mail_put(o + WPV, vx1, tag);
@@ -1068,6 +1073,10 @@ __global__ __launch_bounds__(1024) void k_resident1(const ResArgs<T> r) {
         }
     }
 
+    if (r.nsteps == 1) {                        // the neighbours have loaded their rims
+        if (nit) receive(r.epoch, 0);
+        lds_barrier();
+    }
     if (!r.load || !own) return;
     r.vz[fo + m] = vz;
     r.vx[fo + m] = vx;

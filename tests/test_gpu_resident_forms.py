@@ -1,0 +1,64 @@
+"""The resident propagation where a launch, a tiling or a batch takes another form than in
+test_gpu_resident.py.
+
+Checkpoints, kept units and the batch's split cut the same time steps of the same arithmetic
+into other launches, so those comparisons are bit for bit.
+"""
+import numpy as np
+import pytest
+
+import cases
+from conftest import gpu_available
+
+pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not gpu_available(), reason="needs a GPU")]
+
+
+@pytest.fixture(scope="module")
+def O():
+    from oracle import oracle as O_
+    O_.load("oracle")
+    return O_
+
+
+@pytest.fixture(scope="module")
+def psv():
+    from fwi_cuda_amd import psv as P
+    return P
+
+
+def _obs(c, seed=5):
+    """Observed rows of about the synthetics' size."""
+    n = len(c["z_rec"]) * int(c["nshot"])
+    rng = np.random.default_rng(seed)
+    t = np.arange(int(c["nt"]))
+    w = np.exp(-(((t - 0.4 * c["nt"]) / (0.1 * c["nt"] + 1)) ** 2))
+    return [1e-13 * rng.standard_normal((n, 1)) * w for _ in range(2)]
+
+
+# nz, nx, order, shots: several tiles of the one-exchange kernel, a last unit of one step
+ONE_STEP = [(90, 140, 8, 2), (91, 139, 10, 3), (201, 401, 8, 1), (97, 133, 12, 1)]
+
+
+@pytest.mark.parametrize("nt", [1, 2, 61])
+@pytest.mark.parametrize("form", ONE_STEP, ids=lambda f: f"{f[0]}x{f[1]}-o{f[2]}x{f[3]}")
+def test_one_step_launches_bitwise(psv, O, form, nt):
+    """Launches of a single time step (a last unit of one step, units of one step, a record of
+    one step) give the bits of one launch over all steps."""
+    nz, nx, order, ns = form
+    c = cases.small_case(O, nz=nz, nx=nx, nt=nt, fdorder=order, nshot=ns, snap_dt=1)
+    obs = _obs(c)
+    out = []
+    for kw in (dict(storage=psv._lib.STORE_FULL), dict(storage=psv._lib.STORE_CHECKPOINT, ckpt_interval=12, ckpt_keep=1),
+               dict(storage=psv._lib.STORE_CHECKPOINT, ckpt_interval=1, ckpt_keep=1),
+               dict(storage=psv._lib.STORE_CHECKPOINT, ckpt_interval=4, ckpt_keep=2, ckpt_slots=3)):
+        with psv.Simulation(c, **kw) as sim:
+            seis = sim.forward()
+            wf = sim.wavefield(0, "szx")
+            sim.set_observed(*obs)
+            m = sim.gradient()
+            out.append((*seis, wf, m, *sim.get_gradient(), *sim.misfit_gradient(*obs), *sim.misfit_gradient_exact(*obs)))
+        print(f"{form} nt {nt} {kw}", flush=True)
+    assert nt < 61 or all(np.abs(a).max() > 0 for a in out[0])
+    for o in out[1:]:
+        for i, (a, b) in enumerate(zip(o, out[0])):
+            np.testing.assert_array_equal(a, b, err_msg=str(i))
