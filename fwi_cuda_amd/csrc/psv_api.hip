@@ -144,7 +144,6 @@ struct fwi_ctx {
     bool plain = false;
     PlainBufs pb{};
     bool tuned = false;
-    int tuned_nb = 0;   // the batch it was tuned for
     int var = 2;   // stencil kernel variant (autotuned); 4 = one-pass step
     int order = 0; // stencil work order (autotuned)
     int depth = 1; // rows the one-pass step loads ahead (autotuned)
@@ -708,11 +707,13 @@ class ChunkGraph {
     hipGraphExec_t exec_ = nullptr;
 };
 
-int zero_state(fwi_ctx *c, int nb, const Wave &w, bool u_we) {
+// zero state of nb shots; level2: also the one-pass step's second level, which the resident
+// kernels do not have
+int zero_state(fwi_ctx *c, int nb, const Wave &w, bool u_we, bool level2) {
     for (int i = 0; i < 5; ++i) HIPCHK(hipMemsetAsync(w.f[i], 0, sizeof(float) * nb * c->fs(), c->st));
     for (int i = 0; i < 4; ++i) HIPCHK(hipMemsetAsync(w.psi[i], 0, sizeof(float) * nb * c->psiz(), c->st));
     for (int i = 4; i < 8; ++i) HIPCHK(hipMemsetAsync(w.psi[i], 0, sizeof(float) * nb * c->psix(), c->st));
-    if (c->fusable && !resident(c, nb)) {   // the one-pass step never writes cells outside the interior: keep them zero
+    if (c->fusable && level2) {   // the one-pass step never writes cells outside the interior: keep them zero
         for (int i = 0; i < 5; ++i) HIPCHK(hipMemsetAsync(w.f2[i], 0, sizeof(float) * nb * c->fs(), c->st));
         for (int i = 0; i < 2; ++i) HIPCHK(hipMemsetAsync(w.psi2[i], 0, sizeof(float) * nb * c->psiz(), c->st));
         for (int i = 2; i < 4; ++i) HIPCHK(hipMemsetAsync(w.psi2[i], 0, sizeof(float) * nb * c->psix(), c->st));
@@ -757,13 +758,14 @@ int check_finite(fwi_ctx *c, int nb) {
 }
 
 // Autotuner: kernel variant, rows per thread (TZ) and work order of the two
-// stencil kernels, timed on the batch (zeroed state, a few steps per candidate);
-// the best is kept per (grid, order, batch) for the process.
+// stencil kernels, timed on a gradient's batch (zeroed state, a few steps per candidate);
+// the best is kept per (grid, order, batch) for the process, and a context keeps what its
+// first pass got for all its passes, whatever their number of shots: a gradient's batches, its
+// misfit and the trials it is compared with then come from one kernel.
 struct TuneKey {
     int nz, nx, N, B;
-    bool fwd;
     bool operator<(const TuneKey &o) const {
-        return std::tie(nz, nx, N, B, fwd) < std::tie(o.nz, o.nx, o.N, o.B, o.fwd);
+        return std::tie(nz, nx, N, B) < std::tie(o.nz, o.nx, o.N, o.B);
     }
 };
 struct TuneVal {
@@ -772,21 +774,18 @@ struct TuneVal {
 std::map<TuneKey, TuneVal> g_tuned;
 std::mutex g_tune_mu;
 
-void take(fwi_ctx *c, const TuneVal &v, int nb) {
+void take(fwi_ctx *c, const TuneVal &v) {
     c->var = v.var;
     c->tz = v.tz;
     c->depth = v.depth;
     c->order = v.order;
     c->tuned = true;
-    c->tuned_nb = nb;
 }
 
-int autotune(fwi_ctx *c, int nb) {
-    if (c->plain || resident(c, nb) || (c->tuned && c->tuned_nb == nb)) return FWI_OK;
-    // a forward batch larger than a gradient's is tuned by forward steps alone: snapshots and
-    // sums hold a gradient's batch only
-    const bool fwd = nb > c->Bg;
-    const TuneKey key{c->g.nz, c->g.nx, c->N, nb, fwd};
+int autotune(fwi_ctx *c) {
+    if (c->plain || c->tuned) return FWI_OK;
+    const int nb = c->Bg;   // what the snapshots and sums hold
+    const TuneKey key{c->g.nz, c->g.nx, c->N, nb};
     const int fv = c->o.kernel_variant;   // 0 = any
     const bool order_forced = c->o.work_order >= 1 && c->o.work_order <= 4;
     // candidates (variant, rows per segment, prefetch depth); the one-pass step only where it applies
@@ -824,7 +823,7 @@ int autotune(fwi_ctx *c, int nb) {
                                    "variant 4's conditions and variant 6's z CPML strips)"
                                  : "");
     if (cand.size() == 1 && order_forced) {   // nothing left to choose
-        take(c, {cand[0].var, cand[0].tz, cand[0].depth, c->o.work_order - 1}, nb);
+        take(c, {cand[0].var, cand[0].tz, cand[0].depth, c->o.work_order - 1});
         return FWI_OK;
     }
     {
@@ -833,12 +832,12 @@ int autotune(fwi_ctx *c, int nb) {
         if (it != g_tuned.end() && (!fv || fv == it->second.var) && (!one_pass(it->second.var) || c->fusable) &&
             (!order_forced || c->o.work_order - 1 == it->second.order) &&
             (c->o.tile_tz <= 0 || c->o.tile_tz == it->second.tz)) {
-            take(c, it->second, nb);
+            take(c, it->second);
             return FWI_OK;
         }
     }
     const Wave w = main_wave(c);
-    RETIF(zero_state(c, nb, w, true));
+    RETIF(zero_state(c, nb, w, true, true));
     KArgs a = base_args(c, nb, w);   // the one-pass step reads f and writes f2 on every repetition
     a.energy = 1;
     hipEvent_t e0, e1;
@@ -866,8 +865,8 @@ int autotune(fwi_ctx *c, int nb) {
     ap.displ = 1;
     std::vector<KArgs *> mix;
     for (int k = 0; k < kmix; ++k) mix.push_back(&a);
-    for (int k = 0; k < kmix && !fwd; ++k) mix.push_back(k ? &ar : &as);
-    for (int k = 0; k < kmix && !fwd; ++k) mix.push_back(k ? &ap : &ag);
+    for (int k = 0; k < kmix; ++k) mix.push_back(k ? &ar : &as);
+    for (int k = 0; k < kmix; ++k) mix.push_back(k ? &ap : &ag);
     auto run = [&](const TuneVal &v) {
         for (KArgs *x : mix) {
             x->order = a.order;
@@ -905,7 +904,7 @@ int autotune(fwi_ctx *c, int nb) {
     }
     hipEventDestroy(e0);
     hipEventDestroy(e1);
-    take(c, bv, nb);
+    take(c, bv);
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tuned[key] = bv;
     return FWI_OK;
@@ -913,9 +912,10 @@ int autotune(fwi_ctx *c, int nb) {
 
 // Forward pass (kernel_PSV with grad = false) for shots [s0, s0 + nb).
 int run_forward(fwi_ctx *c, int s0, int nb, bool store, bool record, bool energy) {
-    RETIF(autotune(c, nb));
+    const bool res = resident(c, nb);
+    if (!res) RETIF(autotune(c));
     const Wave w = main_wave(c);
-    RETIF(zero_state(c, nb, w, true));
+    RETIF(zero_state(c, nb, w, true, !res));
     if (record) HIPCHK(hipMemsetAsync(c->acc, 0, sizeof(double) * 2 * c->nrec_tot, c->st));
     KArgs a = base_args(c, nb, w);
     a.energy = energy;
@@ -932,7 +932,6 @@ int run_forward(fwi_ctx *c, int s0, int nb, bool store, bool record, bool energy
     // snapshots go to slab (it - tb) / snap_dt: every step with full storage, from t_keep
     // (a unit boundary) on with checkpoints
     const int tb = ckpt ? c->t_keep : 0;
-    const bool res = resident(c, nb);
     for (int it = 0; it < nt;) {
         if (ckpt && it % c->S == 0 && c->spine_slot[it / c->S] >= 0) {
             Timer t(c, FWI_K_STORE);
@@ -1038,8 +1037,9 @@ void flush_sums_at(fwi_ctx *c, int nb, int k) {
 // Adjoint pass (kernel_PSV with grad = true): residuals in res_* are injected at
 // the receivers in reversed time, each shot's scaled by its alpha (a power of two).
 int run_adjoint(fwi_ctx *c, int s0, int nb) {
+    const bool res = resident(c, nb);
     const Wave w = main_wave(c);
-    RETIF(zero_state(c, nb, w, false));
+    RETIF(zero_state(c, nb, w, false, !res));
     for (int i = 5; i < 7; ++i) HIPCHK(hipMemsetAsync(c->f[i], 0, sizeof(float) * nb * c->fs(), c->st));
     HIPCHK(hipMemsetAsync(c->f[8], 0, sizeof(float) * nb * c->fs(), c->st));
     for (int i = 0; i < 3; ++i)
@@ -1058,7 +1058,6 @@ int run_adjoint(fwi_ctx *c, int s0, int nb) {
     ag.si_base = c->si_base;
     ag.si_dir = -1;
     ChunkGraph cga(c);
-    const bool res = resident(c, nb);
     if (c->storage != FWI_STORE_CHECKPOINT && res) {
         RETIF(resident_steps(c, s0, nb, w, nt - 1, nt, -1, c->f[8], false, 0, false));
         if (nt % kFlushSteps) flush_sums(c, nb);
@@ -1085,7 +1084,7 @@ int run_adjoint(fwi_ctx *c, int s0, int nb) {
         if (nt % kFlushSteps) flush_sums(c, nb);
     } else {
         const Wave rw = recompute_wave(c);
-        RETIF(zero_state(c, nb, rw, false));   // cells outside the interior stay zero in both levels
+        RETIF(zero_state(c, nb, rw, false, !res));   // cells outside the interior stay zero in both levels
         KArgs r = base_args(c, nb, rw);
         const SrcArgs fsa = src_args(c, s0, nb);
         KArgs rg = r;   // recomputed steps of a replayed graph: time index base + k
@@ -1101,7 +1100,7 @@ int run_adjoint(fwi_ctx *c, int s0, int nb) {
         // a short last segment that left it swapped agree
         auto restore = [&](int hold) -> int {
             if (rw.f[0] != c->rf_canon) rw.flip();
-            if (hold < 0) return zero_state(c, nb, rw, false);
+            if (hold < 0) return zero_state(c, nb, rw, false, !res);
             Timer t(c, FWI_K_STORE);
             return ckpt_copy(c, hold, nb, rw, false);
         };

@@ -62,3 +62,21 @@ def test_one_step_launches_bitwise(psv, O, form, nt):
     for o in out[1:]:
         for i, (a, b) in enumerate(zip(o, out[0])):
             np.testing.assert_array_equal(a, b, err_msg=str(i))
+
+
+def test_tuned_once_per_context(psv, O):
+    """The stencil kernel is tuned once: batches of other sizes (11 shots as 4 + 4 + 3, sub-ranges)
+    keep the choice, also after a context with a pinned variant has tuned the same sizes."""
+    c = cases.small_case(O, nz=89, nx=143, nt=20, nshot=11, snap_dt=1)
+    with psv.Simulation(c, batch=4, work_order=1) as sim:   # a pinned order: launch by launch
+        sim.set_observed(*_obs(c))
+        sim.forward()
+        log = sim.tuning()[1]
+        assert log.startswith("chosen") and log.count("o0/v5/tz16/d1 ") == 1
+        for other in (1, 2):   # one of them at least is not its choice
+            with psv.Simulation(c, batch=4, kernel_variant=other) as pinned:
+                pinned.forward(0, 3)
+                pinned.forward(0, 4)
+            for call in (lambda: sim.forward(0, 3), lambda: sim.gradient(0, 4), lambda: sim.gradient(), lambda: sim.misfit()):
+                call()
+                assert sim.tuning()[1] == log
