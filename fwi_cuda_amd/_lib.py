@@ -85,6 +85,7 @@ def load() -> C.CDLL:
         "fwi_create": (C.c_int32, [C.POINTER(FwiGrid), C.POINTER(FwiAcq), C.POINTER(FwiOpts), C.POINTER(vp)]),
         "fwi_destroy": (None, [vp]),
         "fwi_plan": (C.c_int32, [vp, _ip, _ip, _ip, C.POINTER(C.c_int64)]),
+        "fwi_gradient_batch": (C.c_int32, [vp, _ip]),
         "fwi_checkpoint_plan": (C.c_int32, [vp, _ip, _ip, _dp]),
         "fwi_checkpoint_kept": (C.c_int32, [vp, _ip]),
         "fwi_set_model_device": (C.c_int32, [vp, vp, vp, vp]),
@@ -159,4 +160,5 @@ EXPORTED = ("fwi_abi_version", "fwi_strerror", "fwi_last_error", "fwi_default_op
             "fwi_taper_gradient", "fwi_misfit", "fwi_save_model", "fwi_update_model", "fwi_step_length",
             "fwi_iteration", "fwi_tuning", "fwi_profile", "fwi_profile_kernels", "fwi_profile_stride", "fwi_kernel_times", "fwi_sync", "fwi_forward_snapshots",
             "fwi_mat_av2_noalloc", "fwi_checkpoint_plan", "fwi_checkpoint_kept", "fwi_set_model_device", "fwi_forward_device",
-            "fwi_misfit_gradient_device", "fwi_misfit_gradient_exact", "fwi_pcg_direction", "fwi_smooth_gradient")
+            "fwi_misfit_gradient_device", "fwi_misfit_gradient_exact", "fwi_pcg_direction", "fwi_smooth_gradient",
+            "fwi_gradient_batch")

@@ -2035,6 +2035,12 @@ int32_t fwi_plan(const fwi_ctx *c, int32_t *batch, int32_t *storage, int32_t *ck
     return FWI_OK;
 }
 
+int32_t fwi_gradient_batch(const fwi_ctx *c, int32_t *batch) {
+    if (!c) return FWI_EINVAL;
+    if (batch) *batch = c->Bg;
+    return FWI_OK;
+}
+
 int32_t fwi_checkpoint_plan(const fwi_ctx *c, int32_t *units, int32_t *slots, double *recompute) {
     if (!c) return FWI_EINVAL;
     const bool ck = c->storage == FWI_STORE_CHECKPOINT;

@@ -232,9 +232,10 @@ class Simulation:
         self._chk(self.lib.fwi_plan(self.ctx, C.byref(b), C.byref(s), C.byref(k), C.byref(n)))
         u, sl, rf = C.c_int32(), C.c_int32(), C.c_double()
         self._chk(self.lib.fwi_checkpoint_plan(self.ctx, C.byref(u), C.byref(sl), C.byref(rf)))
-        kept = C.c_int32()
+        kept, bg = C.c_int32(), C.c_int32()
+        self._chk(self.lib.fwi_gradient_batch(self.ctx, C.byref(bg)))
         self._chk(self.lib.fwi_checkpoint_kept(self.ctx, C.byref(kept)))
-        return dict(batch=b.value, storage={1: "full", 2: "checkpoint"}.get(s.value, s.value),
+        return dict(batch=b.value, gradient_batch=bg.value, storage={1: "full", 2: "checkpoint"}.get(s.value, s.value),
                     ckpt_interval=k.value, device_bytes=n.value, ckpt_units=u.value, ckpt_slots=sl.value,
                     ckpt_kept=kept.value, recompute=round(rf.value, 4))
 

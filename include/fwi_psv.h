@@ -121,7 +121,8 @@ typedef struct {
 } fwi_acq;
 
 typedef struct {
-    int32_t batch;          /* shots advanced together in one launch; 0 = as many as memory allows.
+    int32_t batch;          /* shots advanced together in one launch; 0 = as many as memory allows
+                               (with AUTO storage a gradient may take fewer, fwi_gradient_batch).
                                With CHECKPOINT storage a smaller batch leaves memory for more kept
                                units (ckpt_keep); at 1001 x 2001, 8 shots per launch fill the GPU */
     int32_t storage;        /* enum fwi_storage */
@@ -230,9 +231,15 @@ double fwi_dtstab(int32_t nz, int32_t nx, double dh, int32_t fw, const double *r
 /* ---- context ----------------------------------------------------------------- */
 int32_t fwi_create(const fwi_grid *grid, const fwi_acq *acq, const fwi_opts *opts, fwi_ctx **out);
 void fwi_destroy(fwi_ctx *ctx);
-/* Batch size and storage the context chose, and its device memory in bytes. */
+/* Shots of a forward pass's batch and the storage the context chose, and its device memory in
+ * bytes.  The storage is that of a gradient, whose batches may hold fewer shots
+ * (fwi_gradient_batch). */
 int32_t fwi_plan(const fwi_ctx *ctx, int32_t *batch, int32_t *storage, int32_t *ckpt_interval,
                  int64_t *device_bytes);
+/* Shots of a gradient's batch: fwi_plan's batch, or fewer where neither batch nor storage was
+ * given and fewer shots at once spare recomputation.  After a gradient, fwi_get_wavefield
+ * answers for the shots of its last batch. */
+int32_t fwi_gradient_batch(const fwi_ctx *ctx, int32_t *batch);
 
 /* Checkpoint schedule of CHECKPOINT storage: units = segments of ckpt_interval steps,
  * slots = checkpoint buffers, recompute = forward steps run again per time step of the

@@ -80,3 +80,86 @@ def test_tuned_once_per_context(psv, O):
             for call in (lambda: sim.forward(0, 3), lambda: sim.gradient(0, 4), lambda: sim.gradient(), lambda: sim.misfit()):
                 call()
                 assert sim.tuning()[1] == log
+
+
+def test_gradient_batch_smaller_than_forward_batch(psv, O):
+    """With storage and batch left open and memory for part of the snapshots, a gradient runs in
+    smaller batches than a forward pass: same bits as contexts whose one batch holds all shots or
+    that number of shots, and the misfit of a gradient is that of a forward pass."""
+    c = cases.small_case(O, nz=500, nx=700, nt=40, nshot=8, snap_dt=1)
+    kw = dict(kernel_variant=5, tile_tz=16, work_order=1)
+    full = dict(storage=psv._lib.STORE_FULL)
+    with psv.Simulation(c, **kw, **full) as sim:
+        total = sim.plan()["device_bytes"]
+        sim.set_model(1.05 * c["lam"], 1.05 * c["mu"], c["rho"])
+        obs = sim.forward()
+    adj = _obs(c)
+
+    def run(**opts):
+        with psv.Simulation(c, **opts) as sim:
+            plan = sim.plan()
+            seis = sim.forward()
+            sim.set_observed(*obs)
+            m = sim.gradient()
+            assert sum(m.tolist()) == sim.misfit()
+            G, mg = sim.get_gradient(), sim.misfit_gradient(*adj)
+            raw = sim.gradient_raw(*adj)
+            sim.zero_gradient()
+            try:   # its outcome, a step or the search's "no step" exit, and the misfit there
+                it = sim.fwi_iteration()
+            except psv._lib.FwiError as e:
+                it = e.status
+            return (*seis, m, *G, *mg, *raw), plan, (it, sim.misfit())
+
+    for part in (0.9, 0.8, 0.7, 0.6, 0.5):
+        budget = int(part * total)
+        with psv.Simulation(c, mem_budget=budget, **kw) as sim:
+            plan = sim.plan()
+        print(part, plan, flush=True)
+        if plan["gradient_batch"] < plan["batch"] and plan["storage"] == "full":
+            break
+    assert plan["gradient_batch"] < plan["batch"] and plan["device_bytes"] <= budget
+    bg = plan["gradient_batch"]
+    out, p, it = run(mem_budget=budget, **kw)
+    assert p == plan
+    for opts in (full, dict(full, batch=bg), dict(storage=psv._lib.STORE_CHECKPOINT, batch=3)):
+        ref, rp, rit = run(**kw, **opts)
+        assert rp["gradient_batch"] == rp["batch"] and it == rit
+        for i, (a, b) in enumerate(zip(out, ref)):
+            np.testing.assert_array_equal(a, b, err_msg=f"{opts} output {i}")
+    out, p, it = run(mem_budget=budget)   # tuned kernel
+    assert p == plan
+    np.testing.assert_allclose(out[2], ref[2], rtol=1e-5)
+
+
+def test_gradient_batch_over_budgets(psv, O):
+    """The planner's choices over a range of budgets, smaller batches that still checkpoint among
+    them: the bits of one fully stored batch, within the budget."""
+    c = cases.small_case(O, nz=500, nx=700, nt=100, nshot=16, snap_dt=1)
+    obs = _obs(c)
+    kw = dict(kernel_variant=5, tile_tz=16, work_order=1)
+    with psv.Simulation(c, storage=psv._lib.STORE_FULL, **kw) as sim:
+        total = sim.plan()["device_bytes"]
+        sim.set_observed(*obs)
+        want = (sim.gradient(), *sim.get_gradient())
+    seen = set()
+    for k in range(25, 60):
+        budget = int(0.01 * k * total)
+        try:
+            sim = psv.Simulation(c, mem_budget=budget, **kw)
+        except psv._lib.FwiError as e:
+            assert e.status == -2
+            continue
+        with sim:
+            p = sim.plan()
+            key = (p["gradient_batch"], p["batch"], p["storage"])
+            if key in seen:
+                continue
+            seen.add(key)
+            print(k, p, flush=True)
+            assert p["device_bytes"] <= budget
+            sim.set_observed(*obs)
+            got = (sim.gradient(), *sim.get_gradient())
+        for a, b in zip(got, want):
+            np.testing.assert_array_equal(a, b, err_msg=str(p))
+    assert {s for g, b, s in seen if g < b} == {"full", "checkpoint"}
