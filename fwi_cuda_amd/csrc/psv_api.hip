@@ -160,8 +160,8 @@ struct fwi_ctx {
     size_t mail_words = 0;
     uint32_t mail_tag = 1;
     int *res_err = nullptr;
-    char *xws = nullptr;     // the exact adjoint's workspace, kept while it is small (kExactKeep)
-    size_t xws_bytes = 0;
+    char *xws = nullptr;     // the exact adjoint's workspace, kept as ExactRelease allows
+    size_t xws_bytes = 0;    // beside `bytes`
 
     // ---- profiling
     int prof_on = 0, prof_stride = 1;
@@ -2031,7 +2031,7 @@ int32_t fwi_plan(const fwi_ctx *c, int32_t *batch, int32_t *storage, int32_t *ck
     if (batch) *batch = c->B;
     if (storage) *storage = c->storage;
     if (ckpt_interval) *ckpt_interval = c->storage == FWI_STORE_CHECKPOINT ? c->S : 0;
-    if (bytes) *bytes = (int64_t)c->bytes;
+    if (bytes) *bytes = (int64_t)(c->bytes + c->xws_bytes);
     return FWI_OK;
 }
 
@@ -2290,8 +2290,27 @@ int misfit_gradient_dev(fwi_ctx *c, int shot0, int nshots, const double *adj_z, 
 // The exact derivative of J = sum 0.5 dt r^2 (adjoint sources r = adj_z / adj_x, host or
 // device arrays [rows][nt]) with respect to lam, mu, rho into device arrays [nz][nx] (zero
 // outside the snapshot box): the forward run storing its intermediates for every step, the
-// reverse sweep of psv_exact.hip, the media gradient carried through mat_av2.  Its buffers
-// are allocated for the call and freed before it returns; shots go in batches that fit.
+// reverse sweep of psv_exact.hip, the media gradient carried through mat_av2; shots go in
+// batches that fit.  ExactRelease says when the workspace stays with the context.
+
+// At the end of a call, whatever its outcome: the workspace is given back unless it is the
+// resident sweep's and at most kExactKeep bytes, an eighth of the free memory (pool, itself
+// included) and within mem_budget where one is set.
+struct ExactRelease {
+    fwi_ctx *c;
+    size_t pool;
+    bool res;
+    ~ExactRelease() {
+        (void)hipStreamSynchronize(c->st);
+        if (res && c->xws_bytes <= std::min(kExactKeep, pool / 8) &&
+            (c->o.mem_budget <= 0 || c->bytes + c->xws_bytes <= (size_t)c->o.mem_budget))
+            return;
+        (void)hipFree(c->xws);
+        c->xws = nullptr;
+        c->xws_bytes = 0;
+    }
+};
+
 int exact_gradient(fwi_ctx *c, int shot0, int nshots, const double *adj_z, const double *adj_x, bool on_device,
                    double *d_lam, double *d_mu, double *d_rho) {
     if (shot0 < 0 || nshots <= 0 || shot0 + nshots > c->nshot) return c->fail(FWI_EINVAL, "shot range");
@@ -2310,7 +2329,8 @@ int exact_gradient(fwi_ctx *c, int shot0, int nshots, const double *adj_z, const
     };
     size_t freeb = 0, total = 0;
     HIPCHK(hipMemGetInfo(&freeb, &total));
-    const size_t avail = (size_t)(0.85 * (double)freeb);
+    const size_t pool = freeb + c->xws_bytes;   // a kept workspace is this call's own
+    const size_t avail = (size_t)(0.85 * (double)pool);
     const size_t g_all = fs * 8 * 5 * (size_t)nshots;   // the media gradients of every shot
     int S = nt;
     if (c->o.storage == FWI_STORE_CHECKPOINT && c->o.ckpt_interval > 0)
@@ -2357,14 +2377,7 @@ int exact_gradient(fwi_ctx *c, int shot0, int nshots, const double *adj_z, const
         }
         c->xws_bytes = ws_bytes;
     }
-    // kept for the next call if it is small beside what is free, else given back
-    auto release = [&]() {
-        (void)hipStreamSynchronize(c->st);
-        if (res && c->xws_bytes <= kExactKeep && c->xws_bytes <= freeb / 8) return;
-        (void)hipFree(c->xws);
-        c->xws = nullptr;
-        c->xws_bytes = 0;
-    };
+    const ExactRelease release{c, pool, res};
     XArgs x{};
     x.nz = nz; x.nx = nx; x.P = c->P; x.B = Bx; x.N = c->N;
     x.pml_z = c->g.pml_z; x.pml_x = c->g.pml_x;
@@ -2537,7 +2550,6 @@ int exact_gradient(fwi_ctx *c, int shot0, int nshots, const double *adj_z, const
                       d_mu, d_rho, c->st);
         r = res ? check_resident(c) : sync(c);
     }
-    release();
     return r;
 }
 

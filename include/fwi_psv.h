@@ -127,7 +127,9 @@ typedef struct {
                                units (ckpt_keep); at 1001 x 2001, 8 shots per launch fill the GPU */
     int32_t storage;        /* enum fwi_storage */
     int32_t ckpt_interval;  /* time steps per checkpoint segment; 0 = chosen from memory */
-    int64_t mem_budget;     /* device bytes the context may allocate; 0 = 90 % of free memory */
+    int64_t mem_budget;     /* device bytes the context may hold; 0 = 90 % of free memory.  The
+                               workspace of fwi_misfit_gradient_exact comes on top during that
+                               call and stays allocated after it only within the budget */
     int32_t form;           /* enum fwi_form */
     int32_t grad_sign;      /* -1 (default): the CPU path's "grad -= ..." (n_kernel_lib_PSV.cpp:477-479);
                                +1: the GPU path's "+=" (d_kernel_lib_PSV.cu:838-840) */
@@ -295,7 +297,9 @@ int32_t fwi_misfit_gradient(fwi_ctx *ctx, int32_t shot0, int32_t nshots, const d
  * running sum) transposed and applied in reverse order, the media gradient taken from the
  * forward's stored strain rates and stress divergences and carried to lam, mu, rho through
  * mat_av2's averages.  Zero outside the snapshot box.  It keeps five fields per time step
- * and shot (FP32) for the call, in batches of shots that fit; on_device: adj_* and the
+ * and shot (FP32) for the call, in batches of shots that fit; on grids that fit the chip the
+ * workspace (at most 8 GiB, an eighth of the free memory and mem_budget) stays with the context
+ * for the next call, counted by fwi_plan; on_device: adj_* and the
  * outputs are device arrays (as in the _device calls below). */
 int32_t fwi_misfit_gradient_exact(fwi_ctx *ctx, int32_t shot0, int32_t nshots, const double *adj_z,
                                   const double *adj_x, double *d_lam, double *d_mu, double *d_rho,

@@ -163,3 +163,25 @@ def test_gradient_batch_over_budgets(psv, O):
         for a, b in zip(got, want):
             np.testing.assert_array_equal(a, b, err_msg=str(p))
     assert {s for g, b, s in seen if g < b} == {"full", "checkpoint"}
+
+
+def test_exact_workspace_counted_and_within_budget(psv, O):
+    """The exact adjoint's workspace stays within mem_budget, is counted by plan(), and a kept one
+    changes neither the next call's result nor its size."""
+    c = cases.small_case(O, nz=90, nx=140, nt=300, nshot=3, snap_dt=1)
+    adj = _obs(c)
+    with psv.Simulation(c) as sim:
+        before = sim.plan()["device_bytes"]
+        a = sim.misfit_gradient_exact(*adj)
+        held = sim.plan()["device_bytes"]
+        assert held - before > 5 * 4 * 90 * 140 * 300 * 3   # the intermediates of every step
+        b = sim.misfit_gradient_exact(*adj)
+        assert sim.plan()["device_bytes"] == held
+    budget = before + (65 << 20)   # the planner's reserve, and less than the workspace
+    with psv.Simulation(c, mem_budget=budget) as sim:
+        d = sim.misfit_gradient_exact(*adj)
+        assert sim.plan()["device_bytes"] <= budget
+    for x, y, z in zip(a, b, d):
+        assert np.abs(x).max() > 0
+        np.testing.assert_array_equal(y, x)
+        np.testing.assert_array_equal(z, x)
