@@ -28,13 +28,20 @@
 // Work split.  A thread owns CPT cells of one column: the z taps of its CPT rows are
 // CPT + 2N - 1 LDS reads per field instead of 2N CPT, the x taps are reads at constant
 // offsets from neighbouring lanes' columns (no bank conflicts).  The arithmetic is that of
-// stencil variant 5, in its order, so results do not depend on the tiling.
+// stencil variant 5, in its order, and every product that is fused into a sum is written so
+// (left to the compiler, a sum of two products fuses the one or the other as a tiling's
+// unrolling has it): results do not depend on the tiling.
 #pragma once
 
 #include "psv_device.h"
 
+#pragma clang fp contract(off)
+
 namespace psv {
 namespace {
+
+__device__ __forceinline__ float fmadd(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fmadd(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
 constexpr int kSpinLimit = 1 << 22;
 
@@ -333,8 +340,8 @@ __global__ __launch_bounds__(1024) void k_resident(const ResArgs<T> r) {
     // p1, p2 of a pass in one direction: the memories of slots j, j + 1 advanced
     auto memory = [&](int j, int k, int z, int xc, T b1, T a1, T d1, T b2, T a2, T d2, T &p1, T &p2) {
         auto advance = [&](T *m1, T *m2) {
-            p1 = b1 * *m1 + a1 * d1;
-            p2 = b2 * *m2 + a2 * d2;
+            p1 = j < 4 ? fmadd(b1, *m1, a1 * d1) : fmadd(a1, d1, b1 * *m1);
+            p2 = j < 4 ? fmadd(b2, *m2, a2 * d2) : fmadd(a2, d2, b2 * *m2);
             *m1 = p1;
             *m2 = p2;
         };
@@ -425,23 +432,23 @@ __global__ __launch_bounds__(1024) void k_resident(const ResArgs<T> r) {
                 T vz_z = 0, vx_z = 0, vz_x = 0, vx_x = 0;
 #pragma unroll
                 for (int i = 1; i <= N; ++i) {
-                    vz_z += r.cz[i - 1] * (qz[k + N + i - 1] - qz[k + N - i]);
-                    vx_z += r.cz[i - 1] * (qx[k + N + i - 1] - qx[k + N - i]);
-                    vz_x += r.cx[i - 1] * (lvz[c + i] - lvz[c + 1 - i]);
-                    vx_x += r.cx[i - 1] * (lvx[c + i - 1] - lvx[c - i]);
+                    vz_z = fmadd(r.cz[i - 1], qz[k + N + i - 1] - qz[k + N - i], vz_z);
+                    vx_z = fmadd(r.cz[i - 1], qx[k + N + i - 1] - qx[k + N - i], vx_z);
+                    vz_x = fmadd(r.cx[i - 1], lvz[c + i] - lvz[c + 1 - i], vz_x);
+                    vx_x = fmadd(r.cx[i - 1], lvx[c + i - 1] - lvx[c - i], vx_x);
                 }
                 if (zin >> k & 1) {
                     const T *pf = zprof + (zv + k) * 6;
                     T p1, p2;
                     memory(0, k, zv, xv, pf[0], pf[1], vz_z, pf[3], pf[4], vx_z, p1, p2);
-                    vz_z = vz_z * pf[2] + p1;
-                    vx_z = vx_z * pf[5] + p2;
+                    vz_z = fmadd(vz_z, pf[2], p1);
+                    vx_z = fmadd(vx_z, pf[5], p2);
                 }
                 if (xin >> k & 1) {
                     T p1, p2;
                     memory(4, k, zv, xv, xb, xa, vx_x, xbh, xah, vz_x, p1, p2);
-                    vx_x = vx_x * xk + p1;
-                    vz_x = vz_x * xkh + p2;
+                    vx_x = fmadd(vx_x, xk, p1);
+                    vz_x = fmadd(vz_x, xkh, p2);
                 }
                 if constexpr (!ADJ && sizeof(T) == 4) {   // the strain rates the reverse sweep reads
                     if (r.hist && k < nc) {
@@ -454,13 +461,13 @@ __global__ __launch_bounds__(1024) void k_resident(const ResArgs<T> r) {
                 }
                 const T l = lam[k], m = mu[k];
                 const T div = l * (vx_x + vz_z);
-                T nzz = lzz[c] + dt * (div + T(2) * m * vz_z);
-                T nzx = lzx[c] + dt * muzx[k] * (vz_x + vx_z);
-                T nxx = lxx[c] + dt * (div + T(2) * m * vx_x);
+                T nzz = fmadd(dt, fmadd(T(2) * m, vz_z, div), lzz[c]);
+                T nzx = fmadd(dt * muzx[k], vz_x + vx_z, lzx[c]);
+                T nxx = fmadd(dt, fmadd(T(2) * m, vx_x, div), lxx[c]);
                 if (k == 0 && top_row) {   // surf_mirror at row N (src/cpu/n_kernel_lib_PSV.cpp:297-301)
                     nzz = 0;
                     nzx = 0;
-                    nxx = T(4) * dt * vx_x * (l * m + m * m) / (l + T(2) * m);
+                    nxx = T(4) * dt * vx_x * fmadd(l, m, m * m) / fmadd(T(2), m, l);
                 }
                 lzz[c] = nzz;
                 lzx[c] = nzx;
@@ -504,24 +511,24 @@ __global__ __launch_bounds__(1024) void k_resident(const ResArgs<T> r) {
                 T szz_z = 0, szx_z = 0, szx_x = 0, sxx_x = 0;
 #pragma unroll
                 for (int i = 1; i <= N; ++i) {
-                    szz_z += r.cz[i - 1] * (qzz[k + N + i - 1] - qzz[k + N - i]);
-                    szx_z += r.cz[i - 1] * (qzx[k + N + i - 1] - qzx[k + N - i]);
-                    szx_x += r.cx[i - 1] * (lzx[c + i - 1] - lzx[c - i]);
-                    sxx_x += r.cx[i - 1] * (lxx[c + i] - lxx[c + 1 - i]);
+                    szz_z = fmadd(r.cz[i - 1], qzz[k + N + i - 1] - qzz[k + N - i], szz_z);
+                    szx_z = fmadd(r.cz[i - 1], qzx[k + N + i - 1] - qzx[k + N - i], szx_z);
+                    szx_x = fmadd(r.cx[i - 1], lzx[c + i - 1] - lzx[c - i], szx_x);
+                    sxx_x = fmadd(r.cx[i - 1], lxx[c + i] - lxx[c + 1 - i], sxx_x);
                 }
                 // the reference's slot mapping (src/cpu/n_kernel_PSV.cpp:142-146)
                 if (zin >> k & 1) {
                     const T *pf = zprof + (zv + k) * 6;
                     T p1, p2;
                     memory(2, k, zv, xv, pf[0], pf[1], szz_z, pf[3], pf[4], szx_z, p1, p2);
-                    szz_z = szz_z * pf[2] + p1;
-                    szx_z = szx_z * pf[5] + p2;
+                    szz_z = fmadd(szz_z, pf[2], p1);
+                    szx_z = fmadd(szx_z, pf[5], p2);
                 }
                 if (xin >> k & 1) {
                     T p1, p2;
                     memory(6, k, zv, xv, xb, xa, sxx_x, xbh, xah, szx_x, p1, p2);
-                    sxx_x = sxx_x * xk + p1;
-                    szx_x = szx_x * xkh + p2;
+                    sxx_x = fmadd(sxx_x, xk, p1);
+                    szx_x = fmadd(szx_x, xkh, p2);
                 }
                 if constexpr (!ADJ && sizeof(T) == 4) {   // the stress divergences
                     if (r.hist && k < nc) {
@@ -532,13 +539,13 @@ __global__ __launch_bounds__(1024) void k_resident(const ResArgs<T> r) {
                     }
                 }
                 const T vz0 = lvz[c], vx0 = lvx[c];
-                const T vz1 = vz0 + dt * rhoz[k] * (szx_x + szz_z);
-                const T vx1 = vx0 + dt * rhox[k] * (sxx_x + szx_z);
+                const T vz1 = fmadd(dt * rhoz[k], szx_x + szz_z, vz0);
+                const T vx1 = fmadd(dt * rhox[k], sxx_x + szx_z, vx0);
                 if constexpr (ADJ) {
-                    uz[k] = uz[k] + dt * vz0;
-                    ux[k] = ux[k] + dt * vx0;
+                    uz[k] = fmadd(dt, vz0, uz[k]);
+                    ux[k] = fmadd(dt, vx0, ux[k]);
                 }
-                if (r.energy) we[k] = we[k] + (vx1 * vx1 + vz1 * vz1);
+                if (r.energy) we[k] = we[k] + fmadd(vx1, vx1, vz1 * vz1);
                 lvz[c] = vz1;
                 lvx[c] = vx1;
                 if constexpr (CPT > 2) __builtin_amdgcn_sched_barrier(0);
@@ -572,20 +579,19 @@ __global__ __launch_bounds__(1024) void k_resident(const ResArgs<T> r) {
                     const T lm = lam[k] + mu[k];
                     const T il = r.gain_lm / (lm * lm), im = r.gain_lm / (mu[k] * mu[k]);
                     const T s1 = T(0.25) * il * (Szz + Sxx) * (c_zz + c_xx);
-                    const T s2 = T(0.25) * im * (Szz - Sxx) * (c_zz - c_xx);
-                    const T s3 = im * (Szx * c_zx);
+                    const T b2 = T(0.25) * im * (Szz - Sxx), d2 = c_zz - c_xx, b3 = Szx * c_zx;
                     auto add = [&](int j, T v) {
-                        if constexpr (kReg) gs[j][k] = gs[j][k] + r.gw * v;
-                        else q->g[j][(size_t)s * slab + lc[k]] = gm[j][k] + r.gw * v;
+                        if constexpr (kReg) gs[j][k] = fmadd(r.gw, v, gs[j][k]);
+                        else q->g[j][(size_t)s * slab + lc[k]] = fmadd(r.gw, v, gm[j][k]);
                     };
                     add(0, s1);
                     if (!r.gform) {
-                        add(1, s3 + s1 + s2);
-                        add(2, ux[k] * Vx + uz[k] * Vz);
+                        add(1, fmadd(b2, d2, fmadd(im, b3, s1)));
+                        add(2, fmadd(uz[k], Vz, ux[k] * Vx));
                     } else {
-                        add(1, s1 + s2);
+                        add(1, s1 + b2 * d2);
                         add(2, dt * (lvz[c] * Vz));
-                        add(3, s3);
+                        add(3, im * b3);
                         add(4, dt * (lvx[c] * Vx));
                     }
                 }
@@ -919,25 +925,25 @@ __global__ __launch_bounds__(1024) void k_resident1(const ResArgs<T> r) {
             T vz_z = 0, vx_z = 0, vz_x = 0, vx_x = 0;
 #pragma unroll
             for (int i = 1; i <= N; ++i) {
-                vz_z += r.cz[i - 1] * (lvz[c + (i - 1) * VW] - lvz[c - i * VW]);
-                vx_z += r.cz[i - 1] * (lvx[c + i * VW] - lvx[c - (i - 1) * VW]);
-                vz_x += r.cx[i - 1] * (lvz[c + i] - lvz[c + 1 - i]);
-                vx_x += r.cx[i - 1] * (lvx[c + i - 1] - lvx[c - i]);
+                vz_z = fmadd(r.cz[i - 1], lvz[c + (i - 1) * VW] - lvz[c - i * VW], vz_z);
+                vx_z = fmadd(r.cz[i - 1], lvx[c + i * VW] - lvx[c - (i - 1) * VW], vx_z);
+                vz_x = fmadd(r.cx[i - 1], lvz[c + i] - lvz[c + 1 - i], vz_x);
+                vx_x = fmadd(r.cx[i - 1], lvx[c + i - 1] - lvx[c - i], vx_x);
             }
             if (zs) {
                 const T *pf = zprof + lz * 6;
-                const T p1 = pf[0] * pr[0] + pf[1] * vz_z, p2 = pf[3] * pr[1] + pf[4] * vx_z;
+                const T p1 = fmadd(pf[0], pr[0], pf[1] * vz_z), p2 = fmadd(pf[3], pr[1], pf[4] * vx_z);
                 pr[0] = p1;
                 pr[1] = p2;
-                vz_z = vz_z * pf[2] + p1;
-                vx_z = vx_z * pf[5] + p2;
+                vz_z = fmadd(vz_z, pf[2], p1);
+                vx_z = fmadd(vx_z, pf[5], p2);
             }
             if (xs) {
-                const T p1 = xb * pr[4] + xa * vx_x, p2 = xbh * pr[5] + xah * vz_x;
+                const T p1 = fmadd(xa, vx_x, xb * pr[4]), p2 = fmadd(xah, vz_x, xbh * pr[5]);
                 pr[4] = p1;
                 pr[5] = p2;
-                vx_x = vx_x * xk + p1;
-                vz_x = vz_x * xkh + p2;
+                vx_x = fmadd(vx_x, xk, p1);
+                vz_x = fmadd(vz_x, xkh, p2);
             }
             if constexpr (!ADJ && sizeof(T) == 4) {
                 if (r.hist && own) {
@@ -948,13 +954,13 @@ __global__ __launch_bounds__(1024) void k_resident1(const ResArgs<T> r) {
                 }
             }
             const T div = lam * (vx_x + vz_z);
-            szz = szz + dt * (div + T(2) * mu * vz_z);
-            szx = szx + dt * muzx * (vz_x + vx_z);
-            sxx = sxx + dt * (div + T(2) * mu * vx_x);
+            szz = fmadd(dt, fmadd(T(2) * mu, vz_z, div), szz);
+            szx = fmadd(dt * muzx, vz_x + vx_z, szx);
+            sxx = fmadd(dt, fmadd(T(2) * mu, vx_x, div), sxx);
             if (top_row) {                      // surf_mirror at row N (src/cpu/n_kernel_lib_PSV.cpp:297-301)
                 szz = 0;
                 szx = 0;
-                sxx = T(4) * dt * vx_x * (lam * mu + mu * mu) / (lam + T(2) * mu);
+                sxx = T(4) * dt * vx_x * fmadd(lam, mu, mu * mu) / fmadd(T(2), mu, lam);
             }
             lzz[d] = szz;
             lzx[d] = szx;
@@ -965,25 +971,25 @@ __global__ __launch_bounds__(1024) void k_resident1(const ResArgs<T> r) {
             T szz_z = 0, szx_z = 0, szx_x = 0, sxx_x = 0;
 #pragma unroll
             for (int i = 1; i <= N; ++i) {
-                szz_z += r.cz[i - 1] * (lzz[d + i * SW] - lzz[d - (i - 1) * SW]);
-                szx_z += r.cz[i - 1] * (lzx[d + (i - 1) * SW] - lzx[d - i * SW]);
-                szx_x += r.cx[i - 1] * (lzx[d + i - 1] - lzx[d - i]);
-                sxx_x += r.cx[i - 1] * (lxx[d + i] - lxx[d + 1 - i]);
+                szz_z = fmadd(r.cz[i - 1], lzz[d + i * SW] - lzz[d - (i - 1) * SW], szz_z);
+                szx_z = fmadd(r.cz[i - 1], lzx[d + (i - 1) * SW] - lzx[d - i * SW], szx_z);
+                szx_x = fmadd(r.cx[i - 1], lzx[d + i - 1] - lzx[d - i], szx_x);
+                sxx_x = fmadd(r.cx[i - 1], lxx[d + i] - lxx[d + 1 - i], sxx_x);
             }
             if (zs) {
                 const T *pf = zprof + lz * 6;
-                const T p1 = pf[0] * pr[2] + pf[1] * szz_z, p2 = pf[3] * pr[3] + pf[4] * szx_z;
+                const T p1 = fmadd(pf[0], pr[2], pf[1] * szz_z), p2 = fmadd(pf[3], pr[3], pf[4] * szx_z);
                 pr[2] = p1;
                 pr[3] = p2;
-                szz_z = szz_z * pf[2] + p1;
-                szx_z = szx_z * pf[5] + p2;
+                szz_z = fmadd(szz_z, pf[2], p1);
+                szx_z = fmadd(szx_z, pf[5], p2);
             }
             if (xs) {
-                const T p1 = xb * pr[6] + xa * sxx_x, p2 = xbh * pr[7] + xah * szx_x;
+                const T p1 = fmadd(xa, sxx_x, xb * pr[6]), p2 = fmadd(xah, szx_x, xbh * pr[7]);
                 pr[6] = p1;
                 pr[7] = p2;
-                sxx_x = sxx_x * xk + p1;
-                szx_x = szx_x * xkh + p2;
+                sxx_x = fmadd(sxx_x, xk, p1);
+                szx_x = fmadd(szx_x, xkh, p2);
             }
             if constexpr (!ADJ && sizeof(T) == 4) {
                 if (r.hist) {
@@ -993,13 +999,13 @@ __global__ __launch_bounds__(1024) void k_resident1(const ResArgs<T> r) {
                 }
             }
             const T vz0 = vz, vx0 = vx;
-            T vz1 = vz0 + dt * rhoz * (szx_x + szz_z);
-            T vx1 = vx0 + dt * rhox * (sxx_x + szx_z);
+            T vz1 = fmadd(dt * rhoz, szx_x + szz_z, vz0);
+            T vx1 = fmadd(dt * rhox, sxx_x + szx_z, vx0);
             if constexpr (ADJ) {
-                uz = uz + dt * vz0;
-                ux = ux + dt * vx0;
+                uz = fmadd(dt, vz0, uz);
+                ux = fmadd(dt, vx0, ux);
             }
-            if (r.energy) we = we + (vx1 * vx1 + vz1 * vz1);
+            if (r.energy) we = we + fmadd(vx1, vx1, vz1 * vz1);
             const T pvz = vz1, pvx = vx1;       // before the injection
             if (gsrc >= 0) {                    // vsrc2: the group's sources in source order
                 const RSeg<T> q = res_seg<T>();
@@ -1036,17 +1042,16 @@ __global__ __launch_bounds__(1024) void k_resident1(const ResArgs<T> r) {
                         const T lm = lam + mu;
                         const T il = r.gain_lm / (lm * lm), im = r.gain_lm / (mu * mu);
                         const T s1 = T(0.25) * il * (Szz + Sxx) * (szz + sxx);
-                        const T s2 = T(0.25) * im * (Szz - Sxx) * (szz - sxx);
-                        const T s3 = im * (Szx * szx);
-                        gs[0] = gs[0] + r.gw * s1;
+                        const T b2 = T(0.25) * im * (Szz - Sxx), d2 = szz - sxx, b3 = Szx * szx;
+                        gs[0] = fmadd(r.gw, s1, gs[0]);
                         if (!r.gform) {
-                            gs[1] = gs[1] + r.gw * (s3 + s1 + s2);
-                            gs[2] = gs[2] + r.gw * (ux * Vx + uz * Vz);
+                            gs[1] = fmadd(r.gw, fmadd(b2, d2, fmadd(im, b3, s1)), gs[1]);
+                            gs[2] = fmadd(r.gw, fmadd(uz, Vz, ux * Vx), gs[2]);
                         } else {
-                            gs[1] = gs[1] + r.gw * (s1 + s2);
-                            gs[2] = gs[2] + r.gw * (dt * (pvz * Vz));
-                            gs[3] = gs[3] + r.gw * s3;
-                            gs[4] = gs[4] + r.gw * (dt * (pvx * Vx));
+                            gs[1] = fmadd(r.gw, s1 + b2 * d2, gs[1]);
+                            gs[2] = fmadd(r.gw, dt * (pvz * Vz), gs[2]);
+                            gs[3] = fmadd(r.gw, im * b3, gs[3]);
+                            gs[4] = fmadd(r.gw, dt * (pvx * Vx), gs[4]);
                         }
                     }
                     if ((r.nt - it) % r.flush_every == 0) {   // the FP32 sums into their FP64 totals

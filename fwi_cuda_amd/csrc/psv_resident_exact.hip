@@ -10,7 +10,8 @@
 // Bound by the exchanges and barriers: 6.3 us a step at 201 x 401, 10 per launch of two
 // shots at 301 x 601.  A call (its forward passes included): 201 x 401, 800 steps 63.5 ->
 // 11.9 ms; 301 x 601, 4 shots, 400 steps 65.6 -> 19.6 ms, both with the workspace kept.
-// Same operations in the same order as psv_exact.hip's kernels, for no free surface or the
+// Same operations in the same order and with the same fused products as psv_exact.hip's
+// kernels, for no free surface or the
 // top one at row N (no image rows) and points inside the interior; other set-ups keep
 // those kernels.
 #include "psv_resident.h"
@@ -130,10 +131,10 @@ __global__ __launch_bounds__(1024) void k_resident_exact(const ResExact r) {
                       float &d2) {
         auto advance = [&](float *m1, float *m2) {
             float q = *m1 + d1;
-            d1 = d1 * k1 + a1 * q;
+            d1 = fmadd(d1, k1, a1 * q);
             *m1 = b1 * q;
             q = *m2 + d2;
-            d2 = d2 * k2 + a2 * q;
+            d2 = fmadd(d2, k2, a2 * q);
             *m2 = b2 * q;
         };
         if constexpr (kPsiReg) {
@@ -194,8 +195,8 @@ __global__ __launch_bounds__(1024) void k_resident_exact(const ResExact r) {
             for (int k = 0; k < CPT; ++k) {
                 const int c = base + k * W;
                 const float az = bvz[k], ax = bvx[k];
-                G[3][k] += (double)az * dt * hs[3][k];
-                G[4][k] += (double)ax * dt * hs[4][k];
+                G[3][k] = fmadd((double)az * dt, (double)hs[3][k], G[3][k]);
+                G[4][k] = fmadd((double)ax * dt, (double)hs[4][k], G[4][k]);
                 const float tz = dt * rhoz[k] * az, tx_ = dt * rhox[k] * ax;
                 float d0 = tz, d2 = tz, d1 = tx_, d3 = tx_;   // szz_z, szx_x; szx_z, sxx_x
                 if (zin >> k & 1) {
@@ -229,10 +230,10 @@ __global__ __launch_bounds__(1024) void k_resident_exact(const ResExact r) {
                 float zz = 0.f, zx = 0.f, xx = 0.f;
 #pragma unroll
                 for (int i = 1; i <= N; ++i) {
-                    zz += r.cz[i - 1] * (q0[k + N - i] - q0[k + N + i - 1]);
-                    zx += r.cz[i - 1] * (q1[k + N - i] - q1[k + N + i - 1]);
-                    zx += r.cx[i - 1] * (l2[c - i + 1] - l2[c + i]);
-                    xx += r.cx[i - 1] * (l3[c - i] - l3[c + i - 1]);
+                    zz = fmadd(r.cz[i - 1], q0[k + N - i] - q0[k + N + i - 1], zz);
+                    zx = fmadd(r.cz[i - 1], q1[k + N - i] - q1[k + N + i - 1], zx);
+                    zx = fmadd(r.cx[i - 1], l2[c - i + 1] - l2[c + i], zx);
+                    xx = fmadd(r.cx[i - 1], l3[c - i] - l3[c + i - 1], xx);
                 }
                 bzz[k] = k < nc ? bzz[k] + zz : 0.f;
                 bzx[k] = k < nc ? bzx[k] + zx : 0.f;
@@ -247,22 +248,23 @@ __global__ __launch_bounds__(1024) void k_resident_exact(const ResExact r) {
                 const int c = base + k * W;
                 float s3 = 0.f;
                 if (k == 0 && top_row) {
-                    const double l = lam[0], u = mu[0], den = l + 2.0 * u;
-                    const double f = (l * u + u * u) / den, f_l = u * u / (den * den),
-                                 f_u = (l * l + 2.0 * l * u + 2.0 * u * u) / (den * den);
+                    const double l = lam[0], u = mu[0], den = fmadd(2.0, u, l);
+                    const double f = fmadd(l, u, u * u) / den, f_l = u * u / (den * den),
+                                 f_u = fmadd(2.0 * u, u, fmadd(l, l, 2.0 * l * u)) / (den * den);
                     const double a = bxx[0], e = hs[1][0];
                     s3 = (float)(a * 4.0 * dt * f);
-                    G[0][0] += a * 4.0 * dt * e * f_l;
-                    G[1][0] += a * 4.0 * dt * e * f_u;
+                    G[0][0] = fmadd(a * 4.0 * dt * e, f_l, G[0][0]);
+                    G[1][0] = fmadd(a * 4.0 * dt * e, f_u, G[1][0]);
                     bzz[0] = bzx[0] = bxx[0] = 0.f;
                 }
                 const float zz = bzz[k], zx = bzx[k], xx = bxx[k];
                 const float e_zz = hs[0][k], e_xx = hs[1][k], e_zx = hs[2][k], l = lam[k], u = mu[k];
-                G[0][k] += (double)dt * ((double)zz + xx) * ((double)e_xx + e_zz);
-                G[1][k] += 2.0 * dt * ((double)zz * e_zz + (double)xx * e_xx);
-                G[2][k] += (double)dt * zx * e_zx;
-                float d0 = dt * ((l + 2.f * u) * zz + l * xx);
-                float d3 = s3 + dt * (l * zz + (l + 2.f * u) * xx);
+                G[0][k] = fmadd((double)dt * ((double)zz + xx), (double)e_xx + e_zz, G[0][k]);
+                G[1][k] = fmadd(2.0 * dt, fmadd((double)zz, (double)e_zz, (double)xx * e_xx), G[1][k]);
+                G[2][k] = fmadd((double)dt * zx, (double)e_zx, G[2][k]);
+                const float lu = fmadd(2.f, u, l);
+                float d0 = dt * fmadd(l, xx, lu * zz);
+                float d3 = fmadd(dt, fmadd(l, zz, lu * xx), s3);
                 float d1 = dt * muzx[k] * zx, d2 = d1;
                 if (zin >> k & 1) {
                     const float *p = zprof + (zv + k) * 6;
@@ -295,10 +297,10 @@ __global__ __launch_bounds__(1024) void k_resident_exact(const ResExact r) {
                 float vz = 0.f, vx = 0.f;
 #pragma unroll
                 for (int i = 1; i <= N; ++i) {
-                    vz += r.cz[i - 1] * (q0[k + N - i] - q0[k + N + i - 1]);
-                    vz += r.cx[i - 1] * (l2[c - i] - l2[c + i - 1]);
-                    vx += r.cz[i - 1] * (q1[k + N - i] - q1[k + N + i - 1]);
-                    vx += r.cx[i - 1] * (l3[c - i + 1] - l3[c + i]);
+                    vz = fmadd(r.cz[i - 1], q0[k + N - i] - q0[k + N + i - 1], vz);
+                    vz = fmadd(r.cx[i - 1], l2[c - i] - l2[c + i - 1], vz);
+                    vx = fmadd(r.cz[i - 1], q1[k + N - i] - q1[k + N + i - 1], vx);
+                    vx = fmadd(r.cx[i - 1], l3[c - i + 1] - l3[c + i], vx);
                 }
                 bvz[k] = k < nc ? bvz[k] + vz : 0.f;
                 bvx[k] = k < nc ? bvx[k] + vx : 0.f;

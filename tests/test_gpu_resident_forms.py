@@ -185,3 +185,35 @@ def test_exact_workspace_counted_and_within_budget(psv, O):
         assert np.abs(x).max() > 0
         np.testing.assert_array_equal(y, x)
         np.testing.assert_array_equal(z, x)
+
+
+# nz, nx, order, shots, steps, free surface: calls on 1, 2, ... of the shots take tilings of their
+# own; the waves are inside the CPML strips before the record ends
+TILINGS = [(246, 335, 8, 6, 250, True), (246, 335, 8, 3, 250, False), (301, 601, 4, 5, 150, False),
+           (90, 140, 12, 3, 300, False), (91, 139, 2, 2, 300, True), (89, 131, 6, 2, 300, False),
+           (93, 121, 10, 2, 300, True), (800, 1400, 8, 1, 100, True)]
+
+
+@pytest.mark.parametrize("form", TILINGS, ids=lambda f: f"{f[0]}x{f[1]}-o{f[2]}-{'surface' if f[5] else 'cpml'}")
+def test_results_do_not_depend_on_the_tiling(psv, O, form):
+    """One shot beside others (adjoint sources of the first shot only), alone, and by variant 5's
+    launches: seismograms, fields, correlation sums and misfit derivative bit for bit, the exact
+    gradient over the tilings."""
+    nz, nx, order, ns, nt, surf = form
+    c = cases.small_case(O, nz=nz, nx=nx, nt=nt, fdorder=order, nshot=ns, surface=surf, snap_dt=2)
+    n = len(c["z_rec"])
+    obs = _obs(c)
+    ref = None
+    for v in (0, 5):
+        with psv.Simulation(c, kernel_variant=v) as sim:
+            for k in range(1, ns + 1) if v == 0 else (ns,):
+                adj = [np.concatenate([o[:n], np.zeros((n * (k - 1), nt))]) for o in obs]
+                out = [s[:n] for s in sim.forward(0, k)]
+                out += [sim.wavefield(0, f) for f in ("vz", "vx", "szz", "szx", "sxx", "We")]
+                out += [*sim.gradient_raw(*adj, 0, k), *sim.misfit_gradient(*adj, 0, k)]
+                out += [*sim.misfit_gradient_exact(*adj, 0, k)]
+                ref = ref or out
+                for i, (a, b) in enumerate(zip(out, ref)):
+                    assert np.abs(b).max() > 0
+                    np.testing.assert_array_equal(a, b, err_msg=f"variant {v}, {k} shots, output {i}: {cases.rel_l2(a, b):.1e}")
+                print(f"{form} variant {v} {k} shots", flush=True)
