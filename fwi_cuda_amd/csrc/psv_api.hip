@@ -2337,27 +2337,37 @@ int exact_gradient(fwi_ctx *c, int shot0, int nshots, const double *adj_z, const
         S = std::min(c->o.ckpt_interval, nt);
     else if (c->o.storage != FWI_STORE_FULL && per_shot_of(nt) + g_all > avail)
         S = std::max(1, std::min(nt, (int)std::lround(std::sqrt(13.0 * nt / 5.0))));
-    // The resident sweep takes no more shots at once, and no more steps per segment, than
-    // kExactKeep holds, and keeps that workspace for the next call: allocating and clearing
-    // the intermediates of all shots and steps anew takes longer than the sweep itself (301 x
-    // 601, 4 shots, 400 steps: 6.2 GB, 155 ms a call against 24), recomputing a segment's
-    // forward steps a fifth of it.
+    // The resident sweep keeps to kExactKeep and keeps that workspace for the next call:
+    // allocating and clearing the intermediates of all shots and steps anew takes longer than
+    // the sweep itself (301 x 601, 4 shots, 400 steps: 6.2 GB, 155 ms a call against 24).  Of
+    // the segmentations that fit, the one of the least step time: more segments recompute more
+    // forward steps but hold more shots at once, which share launches.  Beside the tilings'
+    // model a launch of the sweep measured 2.1 us more a step, a forward one that stores
+    // intermediates 1.0.  Measured in 8 GiB, us a step: 90 x 140, 8 shots, 8000 steps 25.9
+    // unsegmented (3 shots at once), 12.6 in 3 segments (8); 246 x 335, 6 shots, 3000 steps
+    // 63.6 unsegmented (1), 37.4 in 2 segments (3), 39.2 in 6 (6).
     const bool res = resident_plan(c, 1, kResExact) && resident_plan(c, 1, kResExactForward);
-    size_t cap = avail;
+    int Bx = 0;   // shots at once
     if (res && c->o.storage != FWI_STORE_FULL) {
-        cap = std::min(avail, std::max(kExactKeep, g_all + per_shot_of(1)));
-        if (c->o.storage != FWI_STORE_CHECKPOINT || c->o.ckpt_interval <= 0) {
-            int nseg_ = 1;
-            while (per_shot_of((nt + nseg_ - 1) / nseg_) + g_all > cap && nseg_ < 64 && nseg_ < nt) ++nseg_;
-            S = std::min(S, (nt + nseg_ - 1) / nseg_);
+        const bool given = c->o.storage == FWI_STORE_CHECKPOINT && c->o.ckpt_interval > 0;
+        const size_t lim = std::min(avail, kExactKeep);
+        double best = 1e300;
+        for (int k = 1, Smax = S; k <= (given ? 1 : std::min(64, nt)); ++k) {
+            const int S_ = given ? S : std::min(Smax, (nt + k - 1) / k), nseg_ = (nt + S_ - 1) / S_;
+            if (g_all + per_shot_of(S_) > lim) continue;
+            const int b1 = (int)std::min<size_t>((size_t)nshots, (lim - g_all) / per_shot_of(S_));
+            const int nbat = (nshots + b1 - 1) / b1, b = (nshots + nbat - 1) / nbat;
+            const ResPlan &rp = *resident_plan(c, b, kResExact), &fp = *resident_plan(c, b, kResExactForward);
+            const double t = nbat * (rp.us + 2.1 * ((b + rp.shots - 1) / rp.shots) + fp.us +
+                                     1.0 * ((b + fp.shots - 1) / fp.shots) + (1.0 - 1.0 / nseg_) * fp.us);
+            if (t < best) best = t, S = S_, Bx = b;
         }
     }
     const size_t per_shot = per_shot_of(S);
     if (per_shot + g_all > avail)
         return c->fail(FWI_ENOMEM, "the exact adjoint keeps %.2f GB per shot (%d steps of intermediates), %.2f GB free",
                        per_shot / 1e9, S, avail / 1e9);
-    const int Bx = (int)std::max<size_t>(
-        1, std::min<size_t>((size_t)nshots, cap > g_all ? (cap - g_all) / per_shot : 0));
+    if (!Bx) Bx = (int)std::min<size_t>((size_t)nshots, (avail - g_all) / per_shot);
     const int nseg = (nt + S - 1) / S;
     const size_t fl_bytes = sizeof(float) * fs * Bx * 30, hist_bytes = sizeof(float) * fs * Bx * 5 * (size_t)S,
                  G_bytes = sizeof(double) * fs * 5 * nshots,

@@ -222,11 +222,12 @@ void x_media_chain(const XArgs &x, int nb, const double *mu, const double *rho, 
 
 // ---- the resident propagation: many time steps in one launch (psv_resident.h) -----------
 // A tiling: shots per launch, tile size, tiles per shot, cells per thread (0: the kernel of
-// one exchange per step), block and LDS size.
+// one exchange per step), block and LDS size, modelled us of a step of all shots.
 struct ResPlan {
     int shots, TX, TZ, ntx, ntz, cpt, threads;
     int psi_lds, psi_rows, psi_cols;   // CPML memory in LDS: a tile's strip rows and columns, at most
     size_t lds;
+    double us;
 };
 constexpr int kResItems = 4;    // edge values a thread reads per half-step, at most
 constexpr int kRes1Cells = 2;   // cells whose velocities a thread reads per step, at most (cpt 0)

@@ -118,6 +118,7 @@ bool plan_resident(int nz, int nx, int N, int nb, ResUse use, int cus, size_t ld
             }
         }
     }
+    out->us = best;
     return best < (use == kUseStep ? 0.9 * (16.0 + 14.4e-6 * nb * nz * nx) : 1e299);
 }
 

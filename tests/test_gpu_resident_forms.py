@@ -217,3 +217,34 @@ def test_results_do_not_depend_on_the_tiling(psv, O, form):
                     assert np.abs(b).max() > 0
                     np.testing.assert_array_equal(a, b, err_msg=f"variant {v}, {k} shots, output {i}: {cases.rel_l2(a, b):.1e}")
                 print(f"{form} variant {v} {k} shots", flush=True)
+
+
+# nz, nx, shots, steps whose intermediates take more than the 8 GiB that stay with a context, and
+# the shots asked for
+GROUPED = [(246, 335, 3, 2500, (3, 2)), (90, 140, 7, 8000, (7, 5))]
+
+
+@pytest.mark.parametrize("form", GROUPED, ids=lambda f: f"{f[0]}x{f[1]}x{f[2]}")
+def test_exact_grouped_shots_and_segments(psv, O, form):
+    """Records that exceed the kept workspace run in segments and in batches of shots that share
+    launches: the workspace stays bounded, and every call gives the bits of the unsegmented sweep."""
+    nz, nx, ns, nt, counts = form
+    c = cases.small_case(O, nz=nz, nx=nx, nt=nt, nshot=ns, snap_dt=1)
+    n = len(c["z_rec"])
+    adj = _obs(c)
+    kw = dict(storage=psv._lib.STORE_CHECKPOINT, ckpt_keep=1)   # a small context
+    out = {}
+    with psv.Simulation(c, **kw) as sim:                       # the interval is left open
+        base = sim.plan()["device_bytes"]
+        for k in (*counts, *counts):
+            g = sim.misfit_gradient_exact(*[a[:n * k] for a in adj], 0, k)
+            held = sim.plan()["device_bytes"] - base
+            print(form, "shots", k, "held", held >> 20, "MiB", flush=True)
+            assert 0 < held <= (8 << 30) + (16 << 20)          # its output buffer and edge words beside it
+            for a, b in zip(g, out.setdefault(k, g)):
+                np.testing.assert_array_equal(a, b)
+    with psv.Simulation(c, ckpt_interval=nt, **kw) as sim:
+        for k in counts:
+            for a, b in zip(sim.misfit_gradient_exact(*[a[:n * k] for a in adj], 0, k), out[k]):
+                assert np.abs(a).max() > 0
+                np.testing.assert_array_equal(b, a)
