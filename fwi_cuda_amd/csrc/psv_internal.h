@@ -231,7 +231,7 @@ struct ResPlan {
 };
 constexpr int kResItems = 4;    // edge values a thread reads per half-step, at most
 constexpr int kRes1Cells = 2;   // cells whose velocities a thread reads per step, at most (cpt 0)
-constexpr uint32_t res1_words(int TX, int TZ, int wpv) { return (uint32_t)(TX * TZ * 2 * wpv + 15) / 16u * 16u; }
+constexpr uint32_t res1_words(int TX, int TZ) { return (uint32_t)(TX * TZ * 2 + 15) / 16u * 16u; }
 constexpr size_t kResLds = 160 * 1024;   // LDS of a CU
 // columns of a block's lanes (a tile is at most that wide) for a number of cells per thread
 constexpr int res_lanes(int cpt, int elt) { return cpt >= 4 && elt == 4 ? 64 : 32; }

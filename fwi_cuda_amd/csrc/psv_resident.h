@@ -736,10 +736,10 @@ __global__ __launch_bounds__(1024) void k_resident(const ResArgs<T> r) {
 // together: at their cell's place in one array (lines written by several blocks) 17 x 15
 // tiles took 4.4 instead of 3.9; rows of 32 lanes: packed to the tile's width they take
 // fewer wavefronts but 4.0 instead of 3.7.
-template <class T, int N, bool ADJ>
-__global__ __launch_bounds__(1024) void k_resident1(const ResArgs<T> r) {
+template <int N, bool ADJ>
+__global__ __launch_bounds__(1024) void k_resident1(const ResArgs<float> r) {
     extern __shared__ char smem[];
-    constexpr int WPV = (int)sizeof(T) / 4;
+    using T = float;
     constexpr int VA = 32 + 2 * N, VW = 2 * VA, SA = 32, SW = 3 * SA;
     const int t = threadIdx.x, nthr = blockDim.x;
     const int TX = r.TX, TZ = r.TZ;
@@ -826,11 +826,11 @@ __global__ __launch_bounds__(1024) void k_resident1(const ResArgs<T> r) {
     }
 
     // the words this thread reads: velocities of the cells within 2N of the tile
-    const uint32_t tw = res1_words(TX, TZ, WPV), set = gridDim.x * tw;   // words of a tile, of a set
+    const uint32_t tw = res1_words(TX, TZ), set = gridDim.x * tw;   // words of a tile, of a set
     auto word = [&](int cz, int cx) {           // of the cell's owner
         const int ox = (cx - N) / TX, oz = (cz - N) / TZ;
         return (uint32_t)((ls * r.ntz + oz) * r.ntx + ox) * tw +
-               (uint32_t)((cz - N - oz * TZ) * TX + cx - N - ox * TX) * 2u * WPV;
+               (uint32_t)((cz - N - oz * TZ) * TX + cx - N - ox * TX) * 2u;
     };
     uint32_t mw[kRes1Cells];
     int ml[kRes1Cells];
@@ -848,23 +848,22 @@ __global__ __launch_bounds__(1024) void k_resident1(const ResArgs<T> r) {
         ml[q] = rz * VW + rx;
         nit = q + 1;
     }
-    const bool alone = r.ntx * r.ntz == 1;
     const uint32_t mine = own ? word(iz, ix) : 0u;
     bool dead = false;
     auto receive = [&](uint32_t tag, int parity) {
         const RSeg<T> sg = res_seg<T>();
         const unsigned long long *base = sg->mail + (parity ? set : 0u);
-        unsigned long long v[kRes1Cells][2 * WPV];
+        unsigned long long v[kRes1Cells][2];
 #pragma unroll
         for (int q = 0; q < kRes1Cells; ++q)
             if (ml[q] >= 0)
 #pragma unroll
-                for (int j = 0; j < 2 * WPV; ++j) v[q][j] = mail_get(base + mw[q] + j);
+                for (int j = 0; j < 2; ++j) v[q][j] = mail_get(base + mw[q] + j);
 #pragma unroll
         for (int q = 0; q < kRes1Cells; ++q)
             if (ml[q] >= 0) {
 #pragma unroll
-                for (int j = 0; j < 2 * WPV; ++j) {
+                for (int j = 0; j < 2; ++j) {
                     int spin = 0;
                     while ((uint32_t)(v[q][j] >> 32) != tag && !dead) {
                         v[q][j] = mail_get(base + mw[q] + j);
@@ -875,14 +874,7 @@ __global__ __launch_bounds__(1024) void k_resident1(const ResArgs<T> r) {
                     }
                 }
 #pragma unroll
-                for (int f = 0; f < 2; ++f) {
-                    T val;
-                    if constexpr (sizeof(T) == 4)
-                        val = __uint_as_float((uint32_t)v[q][f]);
-                    else
-                        val = __longlong_as_double((long long)((v[q][2 * f] & 0xffffffffull) | v[q][2 * f + WPV - 1] << 32));
-                    lvz[ml[q] + f * VA] = val;
-                }
+                for (int f = 0; f < 2; ++f) lvz[ml[q] + f * VA] = __uint_as_float((uint32_t)v[q][f]);
             }
     };
     auto source_row = [&](int j, int it, T &dz, T &dx) {
@@ -945,7 +937,7 @@ __global__ __launch_bounds__(1024) void k_resident1(const ResArgs<T> r) {
                 vx_x = fmadd(vx_x, xk, p1);
                 vz_x = fmadd(vz_x, xkh, p2);
             }
-            if constexpr (!ADJ && sizeof(T) == 4) {
+            if constexpr (!ADJ) {
                 if (r.hist && own) {
                     T *hp = res_seg<T>()->hist + ((size_t)(it - r.hist_base) * r.hist_B + s) * 5 * r.fs + m;
                     hp[0] = vz_z;
@@ -991,7 +983,7 @@ __global__ __launch_bounds__(1024) void k_resident1(const ResArgs<T> r) {
                 sxx_x = fmadd(sxx_x, xk, p1);
                 szx_x = fmadd(szx_x, xkh, p2);
             }
-            if constexpr (!ADJ && sizeof(T) == 4) {
+            if constexpr (!ADJ) {
                 if (r.hist) {
                     T *hp = res_seg<T>()->hist + (((size_t)(it - r.hist_base) * r.hist_B + s) * 5 + 3) * r.fs + m;
                     hp[0] = szx_x + szz_z;
@@ -1022,10 +1014,10 @@ __global__ __launch_bounds__(1024) void k_resident1(const ResArgs<T> r) {
             vx = vx1;
             lvz[c] = vz1;
             lvx[c] = vx1;
-            if (!alone && (n + 1 < r.nsteps || n == 0)) {
+            if (n + 1 < r.nsteps || n == 0) {
                 unsigned long long *o = res_seg<T>()->mail + (n & 1 ? set : 0u) + mine;
                 mail_put(o, vz1, tag);
-                mail_put(o + WPV, vx1, tag);
+                mail_put(o + 1, vx1, tag);
             }
             if (grec >= 0) {                    // the velocity sample; k_seis_scan makes urec2's running sum
                 const RSeg<T> q = res_seg<T>();
@@ -1104,11 +1096,13 @@ __global__ __launch_bounds__(1024) void k_resident1(const ResArgs<T> r) {
 template <class T, bool ADJ, int N>
 hipError_t launch_resident_n(const ResArgs<T> &r, int cpt, int blocks, int threads, size_t lds, hipStream_t st) {
     constexpr int E = (int)sizeof(T);
-    const void *f = cpt == 0   ? (const void *)k_resident1<T, N, ADJ>
-                    : cpt == 1 ? (const void *)k_resident<T, N, 1, res_lanes(1, E), ADJ>
+    const void *f = cpt == 1   ? (const void *)k_resident<T, N, 1, res_lanes(1, E), ADJ>
                     : cpt == 2 ? (const void *)k_resident<T, N, 2, res_lanes(2, E), ADJ>
-                    : cpt == 4 ? (const void *)k_resident<T, N, 4, res_lanes(4, E), ADJ>
-                               : (const void *)k_resident<T, N, E == 8 ? 4 : 8, res_lanes(E == 8 ? 4 : 8, E), ADJ>;
+                               : (const void *)k_resident<T, N, 4, res_lanes(4, E), ADJ>;
+    if constexpr (E == 4) {
+        if (cpt == 0) f = (const void *)k_resident1<N, ADJ>;
+        if (cpt == 8) f = (const void *)k_resident<T, N, 8, res_lanes(8, E), ADJ>;
+    }
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
     void *args[] = {const_cast<ResArgs<T> *>(&r)};

@@ -74,16 +74,18 @@ bool plan_resident(int nz, int nx, int N, int nb, ResUse use, int cus, size_t ld
             if (TX > 64 || (ntx > 1 && ix - (ntx - 1) * TX < N)) continue;
             const int cols = strip_lines(xmap, N, TX);
             for (int ntz = 1; ntz <= std::min(tiles / ntx, iz); ++ntz) {
-                // one exchange per step; tiles that fill the 32 lanes measured 5 % slower than the
-                // next narrower ones (201 x 401: 24 x 13 cells 3.9 us, 22 x 14 3.7, 16 x 20 3.7)
-                if (use != kUseExact && use != kUseFp64 && TX + 2 * N < 32) {
+                // one exchange per step (a single tile has none: one cell per thread); tiles that
+                // fill the 32 lanes measured 5 % slower than the next narrower ones (201 x 401:
+                // 24 x 13 cells 3.9 us, 22 x 14 3.7, 16 x 20 3.7)
+                if (use != kUseExact && use != kUseFp64 && TX + 2 * N < 32 && ntx * ntz > 1) {
                     const int TZ = (iz + ntz - 1) / ntz;
                     const int thr = (32 * (TZ + 2 * N) + 63) / 64 * 64;
                     if (thr <= 1024 && iz - (ntz - 1) * TZ > 0 &&
                         (TX + 4 * N) * (TZ + 4 * N) <= kRes1Cells * thr) {
-                        // tiles narrower than the frame wait for their neighbours' neighbours too
+                        // tiles narrower than the frame (narrow grids, orders 10 and 12) wait for
+                        // their neighbours' neighbours too
                         const bool thin = (ntx > 1 && TX < 2 * N) || (ntz > 1 && TZ < 2 * N);
-                        const double t = launches * (2.3 - (ntx * ntz == 1 ? 1.2 : 0.0) + (thin ? 0.5 : 0.0) + 1.1e-3 * thr);
+                        const double t = launches * (2.3 + (thin ? 0.5 : 0.0) + 1.1e-3 * thr);
                         if (t < best) {
                             best = t;
                             *out = {g, TX, TZ, ntx, ntz, 0, thr, 0, 0, 0,
@@ -144,7 +146,7 @@ void launch_seis_scan(double *z, double *x, int rows, int nt, double dt, double 
 }
 
 size_t resident_words(const ResPlan &p, int N, int elt) {
-    if (p.cpt == 0) return (size_t)2 * p.shots * p.ntx * p.ntz * res1_words(p.TX, p.TZ, elt / 4);
+    if (p.cpt == 0) return (size_t)2 * p.shots * p.ntx * p.ntz * res1_words(p.TX, p.TZ);
     return (size_t)2 * p.shots * p.ntx * p.ntz * 4 * N * (p.TX + p.TZ) * (elt / 4);
 }
 
