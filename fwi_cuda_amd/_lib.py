@@ -21,6 +21,7 @@ STORE_AUTO, STORE_FULL, STORE_CHECKPOINT = 0, 1, 2
 FORM_FUSED, FORM_PLAIN = 0, 1
 PARAM_LAME, PARAM_VELOCITY = 0, 1
 ABI_VERSION = 6
+PASSES = ("step", "fp64", "exact_forward", "exact")
 KERNELS = ("stress", "velocity", "surface", "source", "receiver", "store", "other", "step", "graph")
 
 
@@ -53,6 +54,11 @@ class FwiOpts(C.Structure):
 
 class FwiKernelTime(C.Structure):
     _fields_ = [("launches", C.c_int64), ("total_ms", C.c_double), ("timed", C.c_int64)]
+
+
+class FwiTiling(C.Structure):
+    _fields_ = [(n, C.c_int32) for n in ("shots", "rows", "cols", "tiles_z", "tiles_x", "cells", "threads", "lds",
+                                         "psi_lds", "psi_rows", "psi_cols")]
 
 
 class FwiError(RuntimeError):
@@ -88,6 +94,8 @@ def load() -> C.CDLL:
         "fwi_gradient_batch": (C.c_int32, [vp, _ip]),
         "fwi_checkpoint_plan": (C.c_int32, [vp, _ip, _ip, _dp]),
         "fwi_checkpoint_kept": (C.c_int32, [vp, _ip]),
+        "fwi_resident_tiling": (C.c_int32, [vp, C.c_int32, C.c_int32, C.POINTER(FwiTiling)]),
+        "fwi_plan_tiling": (C.c_int32, [C.c_int32] * 6 + [_ip, _ip, C.POINTER(FwiTiling)]),
         "fwi_set_model_device": (C.c_int32, [vp, vp, vp, vp]),
         "fwi_forward_device": (C.c_int32, [vp, C.c_int32, C.c_int32, vp, vp]),
         "fwi_misfit_gradient_device": (C.c_int32, [vp, C.c_int32, C.c_int32, vp, vp, vp, vp, vp]),
@@ -161,4 +169,4 @@ EXPORTED = ("fwi_abi_version", "fwi_strerror", "fwi_last_error", "fwi_default_op
             "fwi_iteration", "fwi_tuning", "fwi_profile", "fwi_profile_kernels", "fwi_profile_stride", "fwi_kernel_times", "fwi_sync", "fwi_forward_snapshots",
             "fwi_mat_av2_noalloc", "fwi_checkpoint_plan", "fwi_checkpoint_kept", "fwi_set_model_device", "fwi_forward_device",
             "fwi_misfit_gradient_device", "fwi_misfit_gradient_exact", "fwi_pcg_direction", "fwi_smooth_gradient",
-            "fwi_gradient_batch")
+            "fwi_gradient_batch", "fwi_resident_tiling", "fwi_plan_tiling")

@@ -455,7 +455,10 @@ constexpr int kFlushSteps = 64;   // adjoint steps between flushes of the FP32 c
 // or whose steps the batched kernels run faster (plan_resident).  FP32 steps also keep to a
 // pinned kernel variant, rows per segment or work order; the FP64 propagation and the exact
 // adjoint's passes have no variants.
-enum ResKind { kResStep, kResFp64, kResExactForward, kResExact };
+enum ResKind { kResStep = FWI_PASS_STEP, kResFp64, kResExactForward, kResExact };
+ResUse res_use(ResKind kind) {
+    return kind == kResStep ? kUseStep : kind == kResFp64 ? kUseFp64 : kind == kResExact ? kUseExact : kUseExactForward;
+}
 const ResPlan *resident_plan(fwi_ctx *c, int nb, ResKind kind) {
     if (!c->res_grid || c->plain) return nullptr;
     if (kind == kResStep && (c->o.kernel_variant || c->o.tile_tz > 0 || c->o.work_order)) return nullptr;
@@ -463,9 +466,7 @@ const ResPlan *resident_plan(fwi_ctx *c, int nb, ResKind kind) {
     auto it = cache.find(nb);
     if (it == cache.end()) {
         ResPlan p{};
-        const ResUse use = kind == kResStep ? kUseStep : kind == kResFp64 ? kUseFp64 : kind == kResExact ? kUseExact
-                                                                                             : kUseExactForward;
-        if (!plan_resident(c->g.nz, c->g.nx, c->N, nb, use, c->cus, kResLds, c->zmap_h, c->xmap_h, &p)) p.shots = 0;
+        if (!plan_resident(c->g.nz, c->g.nx, c->N, nb, res_use(kind), c->cus, kResLds, c->zmap_h, c->xmap_h, &p)) p.shots = 0;
         it = cache.emplace(nb, p).first;
     }
     return it->second.shots > 0 ? &it->second : nullptr;
@@ -1732,7 +1733,8 @@ int setup_device(fwi_ctx *c, const fwi_acq *q) {
     c->surf_top_only = c->g.isurf[0] == N && c->g.isurf[1] == 0 && c->g.isurf[2] == 0 && c->g.isurf[3] == 0;
     for (int i = 0; c->fusable && i < c->nsrc_tot; ++i) c->fusable = interior(q->src_z[i], q->src_x[i]);
     for (int i = 0; c->fusable && i < c->nrec_tot; ++i) c->fusable = interior(q->rec_z[i], q->rec_x[i]);
-    {   // the resident propagation: cooperative launches, at most 2^16 - 2 points per shot list
+    {   // the resident propagation: cooperative launches; a group's number + 1 is half of an int, so
+        // surveys of 32767 or more sources or receivers over all shots go launch by launch
         HIPCHK(hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, c->o.device));
         c->zmap_h = zmap;
         c->xmap_h = xmap;
@@ -2054,6 +2056,34 @@ int32_t fwi_checkpoint_plan(const fwi_ctx *c, int32_t *units, int32_t *slots, do
 int32_t fwi_checkpoint_kept(const fwi_ctx *c, int32_t *kept) {
     if (!c) return FWI_EINVAL;
     if (kept) *kept = c->storage == FWI_STORE_CHECKPOINT ? c->keep : 0;
+    return FWI_OK;
+}
+
+namespace {
+void tiling_of(const ResPlan &p, fwi_tiling *t) {
+    *t = {p.shots, p.TZ, p.TX, p.ntz, p.ntx, p.cpt, p.threads, (int32_t)p.lds, p.psi_lds, p.psi_rows, p.psi_cols};
+}
+}  // namespace
+
+int32_t fwi_resident_tiling(fwi_ctx *c, int32_t nshots, int32_t pass, fwi_tiling *t) {
+    if (!c || !t) return FWI_EINVAL;
+    if (nshots < 1 || nshots > c->nshot || pass < FWI_PASS_STEP || pass > FWI_PASS_EXACT)
+        return c->fail(FWI_EINVAL, "tiling of pass %d for %d shots", pass, nshots);
+    const ResPlan *p = resident_plan(c, nshots, (ResKind)pass);
+    tiling_of(p ? *p : ResPlan{}, t);
+    return FWI_OK;
+}
+
+int32_t fwi_plan_tiling(int32_t nz, int32_t nx, int32_t fdorder, int32_t nshots, int32_t pass, int32_t cus,
+                        const int32_t *z_strip, const int32_t *x_strip, fwi_tiling *t) {
+    if (!z_strip || !x_strip || !t || fdorder < 2 || fdorder > 12 || fdorder % 2 || nz <= fdorder || nx <= fdorder ||
+        nshots < 1 || cus < 1 || pass < FWI_PASS_STEP || pass > FWI_PASS_EXACT)
+        return FWI_EINVAL;
+    ResPlan p{};
+    if (!plan_resident(nz, nx, fdorder / 2, nshots, res_use((ResKind)pass), cus, kResLds,
+                       std::vector<int>(z_strip, z_strip + nz), std::vector<int>(x_strip, x_strip + nx), &p))
+        p = ResPlan{};
+    tiling_of(p, t);
     return FWI_OK;
 }
 

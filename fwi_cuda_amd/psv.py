@@ -20,7 +20,7 @@ import ctypes as C
 import numpy as np
 
 from . import _lib
-from ._lib import FwiAcq, FwiGrid, FwiKernelTime, FwiOpts, check, dptr, iptr
+from ._lib import FwiAcq, FwiGrid, FwiKernelTime, FwiOpts, FwiTiling, check, dptr, iptr
 
 # ---------------------------------------------------------------------------
 # preprocessing (src/h_preproc_PSV.cpp, src/h_holbergcoeff.cpp, src/h_checkfd_ssg_elastic.cpp)
@@ -141,6 +141,17 @@ def acquisition_csr(case: dict):
     return src, rec
 
 
+def plan_tiling(nz, nx, fdorder, nshots, kind="step", cus=256, z_strip=None, x_strip=None) -> dict:
+    """The rule of the resident propagation's tilings (fwi_plan_tiling, no device needed): strips are
+    the numbers of the CPML rows / columns from 0, -1 elsewhere."""
+    strips = [np.full(n, -1, np.int32) if s is None else np.ascontiguousarray(s, np.int32)
+              for n, s in ((nz, z_strip), (nx, x_strip))]
+    t = FwiTiling()
+    check(_lib.load().fwi_plan_tiling(int(nz), int(nx), int(fdorder), int(nshots), _lib.PASSES.index(kind), int(cus),
+                                      iptr(strips[0]), iptr(strips[1]), C.byref(t)))
+    return {n: getattr(t, n) for n, _ in t._fields_}
+
+
 class Simulation:
     """One device context: grid, acquisition, model, observed data, gradient.
 
@@ -238,6 +249,14 @@ class Simulation:
         return dict(batch=b.value, gradient_batch=bg.value, storage={1: "full", 2: "checkpoint"}.get(s.value, s.value),
                     ckpt_interval=k.value, device_bytes=n.value, ckpt_units=u.value, ckpt_slots=sl.value,
                     ckpt_kept=kept.value, recompute=round(rf.value, 4))
+
+    def resident_tiling(self, nshots=None, kind="step") -> dict:
+        """The tiling that a pass ("step", "fp64", "exact_forward", "exact") over nshots shots at once
+        takes in this context; shots 0 where it goes launch by launch."""
+        t = FwiTiling()
+        self._chk(self.lib.fwi_resident_tiling(self.ctx, self.nshot if nshots is None else int(nshots),
+                                               _lib.PASSES.index(kind), C.byref(t)))
+        return {n: getattr(t, n) for n, _ in t._fields_}
 
     # -- model (mat_av2) --------------------------------------------------------
     def set_model(self, lam, mu, rho):

@@ -201,6 +201,26 @@ typedef struct {
     int64_t timed;      /* launches that carried events (ABI 6) */
 } fwi_kernel_time;
 
+/* How a pass splits its grid where it keeps a shot in the chip's LDS and runs many time steps
+ * per launch (the resident propagation). */
+typedef struct {
+    int32_t shots;             /* per launch; 0: the pass goes launch by launch */
+    int32_t rows, cols;        /* of a tile (the last ones may be smaller) */
+    int32_t tiles_z, tiles_x;  /* per shot, a block each */
+    int32_t cells;             /* per thread, one above the other; 0: one cell of the tile or of the rim that
+                                  its kernel advances too (one exchange of edges per step instead of two) */
+    int32_t threads, lds;      /* of a block; bytes */
+    int32_t psi_lds;           /* the CPML memories that do not fit registers are in LDS (else in memory) */
+    int32_t psi_rows, psi_cols; /* strip rows and columns of a tile that LDS has room for */
+} fwi_tiling;
+
+enum fwi_pass {
+    FWI_PASS_STEP = 0,          /* FP32 steps: forward, recomputed, adjoint */
+    FWI_PASS_FP64 = 1,          /* the FP64 propagation (seis_fp64) */
+    FWI_PASS_EXACT_FORWARD = 2, /* the exact adjoint's forward steps */
+    FWI_PASS_EXACT = 3          /* its reverse sweep */
+};
+
 enum fwi_kernel_id {
     FWI_K_STRESS = 0,     /* stress half-step (vdiff2 + pml_diff2 + update_s2) */
     FWI_K_VELOCITY = 1,   /* velocity half-step (sdiff2 + pml_diff2 + update_v2 [+ fwi_grad2]) */
@@ -250,6 +270,13 @@ int32_t fwi_gradient_batch(const fwi_ctx *ctx, int32_t *batch);
 int32_t fwi_checkpoint_plan(const fwi_ctx *ctx, int32_t *units, int32_t *slots, double *recompute);
 /* Segments at the end of the time axis whose snapshots the forward pass keeps (ABI 5). */
 int32_t fwi_checkpoint_kept(const fwi_ctx *ctx, int32_t *kept);
+/* The tiling a pass (enum fwi_pass) over nshots shots at once takes in this context. */
+int32_t fwi_resident_tiling(fwi_ctx *ctx, int32_t nshots, int32_t pass, fwi_tiling *tiling);
+/* The rule behind it, without a device: the tiling for a grid, order and number of shots on cus
+ * compute units; z_strip [nz] and x_strip [nx] number the CPML strips' rows and columns from 0
+ * (-1 outside the strips). */
+int32_t fwi_plan_tiling(int32_t nz, int32_t nx, int32_t fdorder, int32_t nshots, int32_t pass, int32_t cus,
+                        const int32_t *z_strip, const int32_t *x_strip, fwi_tiling *tiling);
 
 /* Model lam, mu, rho [nz][nx]; derives mu_zx, rho_zp, rho_xp and the scalar means
  * (mat_av2) on the device. */

@@ -6,9 +6,12 @@ into other launches, so those comparisons are bit for bit.
 """
 import numpy as np
 import pytest
+import torch
 
 import cases
 from conftest import gpu_available
+from test_gpu_resident import _with_outside_receiver
+from test_resident_plan import EXACT_FORMS, FP64_FORMS, STEP_FORMS
 
 pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not gpu_available(), reason="needs a GPU")]
 
@@ -35,8 +38,16 @@ def _obs(c, seed=5):
     return [1e-13 * rng.standard_normal((n, 1)) * w for _ in range(2)]
 
 
+def _ran(sim, kind, want):
+    """The context takes the tiling that the form is there for (on 256 compute units)."""
+    t = sim.resident_tiling(kind=kind)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert {k: t[k] for k in want} == want, t
+    assert t["shots"] > 0
+
+
 # nz, nx, order, shots: several tiles of the one-exchange kernel, a last unit of one step
-ONE_STEP = [(90, 140, 8, 2), (91, 139, 10, 3), (201, 401, 8, 1), (97, 133, 12, 1)]
+ONE_STEP = [(90, 140, 8, 2), (91, 139, 10, 3), (201, 401, 8, 1), (97, 133, 12, 1), (233, 32, 12, 6)]
 
 
 @pytest.mark.parametrize("nt", [1, 2, 61])
@@ -52,6 +63,8 @@ def test_one_step_launches_bitwise(psv, O, form, nt):
                dict(storage=psv._lib.STORE_CHECKPOINT, ckpt_interval=1, ckpt_keep=1),
                dict(storage=psv._lib.STORE_CHECKPOINT, ckpt_interval=4, ckpt_keep=2, ckpt_slots=3)):
         with psv.Simulation(c, **kw) as sim:
+            for kind in ("step", "exact_forward"):
+                _ran(sim, kind, dict(cells=0))
             seis = sim.forward()
             wf = sim.wavefield(0, "szx")
             sim.set_observed(*obs)
@@ -248,3 +261,72 @@ def test_exact_grouped_shots_and_segments(psv, O, form):
             for a, b in zip(sim.misfit_gradient_exact(*[a[:n * k] for a in adj], 0, k), out[k]):
                 assert np.abs(a).max() > 0
                 np.testing.assert_array_equal(b, a)
+
+
+def _form_case(O, form, nt):
+    nz, nx, order, ns, surf, npml = form
+    return cases.small_case(O, nz=nz, nx=nx, nt=nt, fdorder=order, nshot=ns, surface=surf, snap_dt=2,
+                            npml=max(npml, order // 2))
+
+
+def _ids(f):
+    return f"{f[0][0]}x{f[0][1]}-o{f[0][2]}x{f[0][3]}"
+
+
+@pytest.mark.parametrize("form", [f for f in STEP_FORMS if f[1].get("shots") != 0], ids=_ids)
+def test_step_forms_equal_variant5(psv, O, form):
+    """Every kernel and tiling of the FP32 steps, among them the two-exchange kernel of one cell per
+    thread on several tiles, tiles thinner than the frame, a single tile and CPML memories in LDS
+    and in memory: forward and adjoint bit for bit variant 5."""
+    c = _form_case(O, form[0], 120)
+    obs = _obs(c)
+    out = []
+    for v in (5, 0):
+        with psv.Simulation(c, kernel_variant=v) as sim:
+            if v == 0:
+                _ran(sim, "step", form[1])
+            seis = sim.forward()
+            fields = [sim.wavefield(0, f) for f in ("vz", "szx", "We")]
+            sim.set_observed(*obs)
+            m = sim.gradient()
+            out.append((*seis, *fields, m, sim.wavefield(int(c["nshot"]) - 1, "We_adj"), *sim.get_gradient(),
+                        *sim.misfit_gradient(*obs)))
+            assert v == 0 or sim.resident_tiling()["shots"] == 0
+    for i, (a, b) in enumerate(zip(*out)):
+        assert np.abs(a).max() > 0
+        np.testing.assert_array_equal(b, a, err_msg=f"output {i}: {cases.rel_l2(b, a):.1e}")
+
+
+@pytest.mark.parametrize("form", FP64_FORMS, ids=_ids)
+def test_fp64_forms_match_kernels(psv, O, form):
+    """Every tiling of the FP64 propagation against its one-thread-per-cell kernels."""
+    c = _form_case(O, form[0], 100)
+    d, rows, _ = _with_outside_receiver(c)
+    with psv.Simulation(c, seis_fp64=1) as sim:
+        _ran(sim, "fp64", form[1])
+        a = sim.forward()
+    with psv.Simulation(d, seis_fp64=1) as sim:
+        assert sim.resident_tiling(kind="fp64")["shots"] == 0
+        b = sim.forward()
+    for x, y in zip(a, b):
+        assert np.linalg.norm(y[rows]) > 0 and cases.rel_l2(x, y[rows]) < 1e-12
+
+
+@pytest.mark.parametrize("form", EXACT_FORMS, ids=_ids)
+def test_exact_forms_match_kernels(psv, O, form):
+    """Every tiling of the exact adjoint's reverse sweep against its one-thread-per-cell kernels."""
+    c = _form_case(O, form[0], 60)
+    d, rows, n = _with_outside_receiver(c)
+    obs = _obs(c)
+    ext = [np.zeros((n, int(c["nt"]))) for _ in range(2)]
+    for e, o in zip(ext, obs):
+        e[rows] = o
+    with psv.Simulation(c) as sim:
+        _ran(sim, "exact", form[1])
+        a = sim.misfit_gradient_exact(*obs)
+    with psv.Simulation(d) as sim:
+        assert sim.resident_tiling(kind="exact")["shots"] == 0
+        b = sim.misfit_gradient_exact(*ext)
+    for i, (x, y) in enumerate(zip(a, b)):
+        print(f"{form[0]} part {i}: {cases.rel_l2(x, y):.2e}", flush=True)
+        assert np.linalg.norm(y) > 0 and cases.rel_l2(x, y) < 1e-5
