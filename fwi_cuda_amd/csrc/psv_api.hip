@@ -187,6 +187,14 @@ struct fwi_ctx {
         bytes += n * sizeof(T);
         return static_cast<T *>(p);
     }
+    // gives back what dalloc<T>(n) returned; the caller has made sure that nothing uses it
+    template <class T>
+    void dfree(T *p, size_t n) {
+        if (!p) return;
+        allocs.erase(std::find(allocs.begin(), allocs.end(), (void *)p));
+        bytes -= n * sizeof(T);
+        (void)hipFree(p);
+    }
     size_t fs() const { return (size_t)g.nz * P; }
     size_t psiz() const { return (size_t)nzs * P; }
     size_t psix() const { return (size_t)g.nz * nxs; }
@@ -477,9 +485,11 @@ bool resident(fwi_ctx *c, int nb) { return resident_plan(c, nb, kResStep) != nul
 int resident_mail(fwi_ctx *c, const ResPlan &p, int elt, int n, uint32_t *tag) {
     const size_t words = resident_words(p, c->N, elt);
     if (words > c->mail_words) {
-        unsigned long long *m = c->dalloc<unsigned long long>(words);
-        if (!m) return c->fail(FWI_ENOMEM, "edge words of the resident propagation");
-        c->mail = m;
+        RETIF(sync(c));   // launches that use the outgrown ones
+        c->dfree(c->mail, c->mail_words);
+        c->mail_words = 0;
+        c->mail = c->dalloc<unsigned long long>(words);
+        if (!c->mail) return c->fail(FWI_ENOMEM, "edge words of the resident propagation");
         c->mail_words = words;
         c->mail_tag = 0xffffffffu;   // cleared below
     }

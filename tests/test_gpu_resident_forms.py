@@ -330,3 +330,17 @@ def test_exact_forms_match_kernels(psv, O, form):
     for i, (x, y) in enumerate(zip(a, b)):
         print(f"{form[0]} part {i}: {cases.rel_l2(x, y):.2e}", flush=True)
         assert np.linalg.norm(y) > 0 and cases.rel_l2(x, y) < 1e-5
+
+
+def test_outgrown_edge_words_are_given_back(psv, O):
+    """A context that has run ever more shots at once holds the memory of one that ran them all."""
+    c = cases.small_case(O, nz=246, nx=335, nt=20, nshot=6, snap_dt=1)
+    held = []
+    for counts in ((1, 2, 3, 6), (6,)):
+        with psv.Simulation(c) as sim:
+            for k in counts:
+                out = sim.forward(0, k)
+            held.append((sim.plan()["device_bytes"], out))
+    assert held[0][0] == held[1][0]
+    for a, b in zip(held[0][1], held[1][1]):
+        np.testing.assert_array_equal(a, b)
