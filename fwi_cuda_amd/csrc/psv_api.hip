@@ -160,6 +160,7 @@ struct fwi_ctx {
     size_t mail_words = 0;
     uint32_t mail_tag = 1;
     int *res_err = nullptr;
+    bool res_pending = false;   // launched since the flag was read last
     char *xws = nullptr;     // the exact adjoint's workspace, kept as ExactRelease allows
     size_t xws_bytes = 0;    // beside `bytes`
 
@@ -278,23 +279,23 @@ void prof_collect(fwi_ctx *c) {
     prof_take(c, c->ev_pending.size());
 }
 
+// a resident launch's wait that gave up (none does while every block is resident)
+int resident_gave_up(fwi_ctx *c) {
+    HIPCHK(hipMemsetAsync(c->res_err, 0, sizeof(int), c->st));
+    return c->fail(FWI_EHIP, "resident propagation: a tile's neighbour did not answer");
+}
+
+// waits for the stream; after resident launches also reads their flag
 int sync(fwi_ctx *c) {
+    int gave_up = 0;
+    if (c->res_pending) HIPCHK(hipMemcpyAsync(&gave_up, c->res_err, sizeof(int), hipMemcpyDeviceToHost, c->st));
     hipError_t e = hipStreamSynchronize(c->st);
     if (e != hipSuccess) return c->fail(FWI_EHIP, "stream: %s", hipGetErrorString(e));
     e = hipGetLastError();
     if (e != hipSuccess) return c->fail(FWI_EHIP, "launch: %s", hipGetErrorString(e));
     prof_collect(c);
-    return FWI_OK;
-}
-
-// after resident launches: a wait that gave up (none does while every block is resident)
-int check_resident(fwi_ctx *c) {
-    int h = 0;
-    HIPCHK(hipMemcpyAsync(&h, c->res_err, sizeof(int), hipMemcpyDeviceToHost, c->st));
-    RETIF(sync(c));
-    if (!h) return FWI_OK;
-    HIPCHK(hipMemsetAsync(c->res_err, 0, sizeof(int), c->st));
-    return c->fail(FWI_EHIP, "resident propagation: a tile's neighbour did not answer");
+    c->res_pending = false;
+    return gave_up ? resident_gave_up(c) : FWI_OK;
 }
 
 template <class T>
@@ -499,6 +500,7 @@ int resident_mail(fwi_ctx *c, const ResPlan &p, int elt, int n, uint32_t *tag) {
     }
     *tag = c->mail_tag;
     c->mail_tag += (uint32_t)n + 1u;
+    c->res_pending = true;
     return FWI_OK;
 }
 
@@ -756,14 +758,15 @@ int ckpt_copy(fwi_ctx *c, int k, int nb, const Wave &w, bool save) {
 }
 
 int check_finite(fwi_ctx *c, int nb) {
-    if (!c->o.check_finite) return resident(c, nb) ? check_resident(c) : FWI_OK;
+    if (!c->o.check_finite) return FWI_OK;
     HIPCHK(hipMemsetAsync(c->nonfinite, 0, sizeof(int), c->st));
     dev_count_nonfinite(c->f[0], nb * c->fs(), c->nonfinite, c->st);
     dev_count_nonfinite(c->f[1], nb * c->fs(), c->nonfinite, c->st);
     int h[2] = {0, 0};   // and the resident propagation's flag
     HIPCHK(hipMemcpyAsync(h, c->nonfinite, 2 * sizeof(int), hipMemcpyDeviceToHost, c->st));
+    c->res_pending = false;
     RETIF(sync(c));
-    if (h[1]) return check_resident(c);
+    if (h[1]) return resident_gave_up(c);
     if (h[0]) return c->fail(FWI_ENONFINITE, "%d non-finite velocity values after propagation", h[0]);
     return FWI_OK;
 }
@@ -1305,7 +1308,7 @@ int run_forward64(fwi_ctx *c, int s0, int nb) {
             HIPCHK(launch_resident_fp64(r, *p, c->N, ns, c->st));
         }
         resident_seismograms(c, s0, nb);
-        return check_resident(c);
+        return FWI_OK;
     }
     int isurf[4];
     for (int k = 0; k < 4; ++k) isurf[k] = c->g.isurf[k];
@@ -2598,7 +2601,7 @@ int exact_gradient(fwi_ctx *c, int shot0, int nshots, const double *adj_z, const
         x.G = G;
         x_media_chain(x, nshots, c->m_mu, c->m_rho, c->g.snap_z1, c->g.snap_z2, c->g.snap_x1, c->g.snap_x2, d_lam,
                       d_mu, d_rho, c->st);
-        r = res ? check_resident(c) : sync(c);
+        r = sync(c);
     }
     return r;
 }

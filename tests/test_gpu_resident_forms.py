@@ -344,3 +344,17 @@ def test_outgrown_edge_words_are_given_back(psv, O):
     assert held[0][0] == held[1][0]
     for a, b in zip(held[0][1], held[1][1]):
         np.testing.assert_array_equal(a, b)
+
+
+def test_without_the_finite_check(psv, O):
+    """check_finite 0 leaves the results of every pass as they are."""
+    c = cases.small_case(O, nz=90, nx=140, nt=150, nshot=3, snap_dt=1)
+    obs = _obs(c)
+    out = []
+    for on in (1, 0):
+        with psv.Simulation(c, check_finite=on, seis_fp64=1) as sim:
+            sim.set_observed(*obs)
+            out.append((*sim.forward(), sim.wavefield(1, "vz"), sim.gradient(), *sim.get_gradient(), sim.misfit(),
+                        *sim.misfit_gradient(*obs), *sim.misfit_gradient_exact(*obs)))
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(b, a)
