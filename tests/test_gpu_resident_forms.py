@@ -358,3 +358,43 @@ def test_without_the_finite_check(psv, O):
                         *sim.misfit_gradient(*obs), *sim.misfit_gradient_exact(*obs)))
     for a, b in zip(*out):
         np.testing.assert_array_equal(b, a)
+
+
+def test_contexts_on_several_threads(psv, O):
+    """Contexts that run resident launches at the same time, each on its own thread and stream,
+    beside one that goes launch by launch: the results of one after the other."""
+    import threading
+    forms = [(90, 140, 8, 2, {}), (246, 335, 8, 3, {}), (301, 601, 4, 2, {}), (90, 140, 8, 2, dict(kernel_variant=5))]
+    work = []
+    for nz, nx, order, ns, kw in forms:
+        c = cases.small_case(O, nz=nz, nx=nx, nt=150, fdorder=order, nshot=ns, snap_dt=1)
+        work.append((psv.Simulation(c, **kw), _obs(c)))
+
+    def run(sim, obs):
+        sim.set_observed(*obs)
+        sim.zero_gradient()
+        return (*sim.forward(), sim.gradient(), *sim.get_gradient(), *sim.misfit_gradient_exact(*obs))
+
+    want = [run(*w) for w in work]
+    got, errors = [[] for _ in work], []
+
+    def loop(i):
+        try:
+            for _ in range(4):
+                got[i].append(run(*work[i]))
+        except Exception as e:   # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=loop, args=(i,)) for i in range(len(work))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for sim, _ in work:
+        sim.close()
+    assert not errors, errors
+    for w, runs in zip(want, got):
+        assert len(runs) == 4
+        for r in runs:
+            for a, b in zip(r, w):
+                np.testing.assert_array_equal(a, b)
