@@ -202,6 +202,17 @@ def measured_traffic(inst, algo_bytes, path=None, rtol=0.01):
     return None
 
 
+def resident_report(tiling, N, avg_ms, launches, timed, time_steps):
+    """The roofline entry where the stencil is the resident propagation: a launch advances a whole
+    range of time steps with the fields on the chip, so its time is given per time step of the
+    batch and no HBM bandwidth is made of it."""
+    c, lanes = tiling["cells"], 64 if tiling["cells"] >= 4 else 32
+    return {"kernel": "step", "instantiation": f"k_resident1<{N}, *>" if c == 0 else f"k_resident<float, {N}, {c}, {lanes}, *>",
+            "bound": "edge exchange and issue (the fields stay on the chip)", "achieved": None, "peak": None, "frac": None,
+            "traffic": None, "avg_launch_ms": round(avg_ms, 4), "launches": launches, "timed_launches": timed,
+            "us_per_time_step": round(avg_ms * launches * 1e3 / max(time_steps, 1), 3), "tiling": tiling}
+
+
 class quiet_stdout:
     """Send file descriptor 1 to /dev/null (the reference prints progress from C++)."""
 
@@ -356,8 +367,8 @@ def main():
     kw = dict(batch=sps, tile_tz=args.tile_tz, kernel_variant=args.variant, work_order=args.order,
               storage=storage, ckpt_interval=args.ckpt_interval, ckpt_keep=args.ckpt_keep)
     sim = psv.Simulation(c, **kw)
-    plan = sim.plan()
-    log("plan", plan)
+    plan, tiling = sim.plan(), sim.resident_tiling(sps)
+    log("plan", plan, "resident tiling", tiling)
     # the observed-data forward (it also runs the autotuner) is timed per launch too, so
     # that launch counts and averages can be set beside a profiler's whole-run summary;
     # only the stencil kernels carry events (the roofline's candidates), the small
@@ -451,6 +462,7 @@ def main():
             for k in per_shot_step if kt[k][2] > 0}
     dom = max(kern, key=lambda k: kern[k][1] * kern[k][2])   # the most time: average x launches
     b, avg_ms, n, timed = kern[dom]
+    resident = tiling["shots"] > 0
     achieved = b / n / (avg_ms / 1e3) / 1e9
     # every launch of the run that events timed (the observed-data forward and the timed
     # gradients): the launch set of a whole-run profiler summary of this command
@@ -475,12 +487,14 @@ def main():
                                       "launch, calibrated against a copy kernel, averaged over the gradient's "
                                       "launch mix (forward, recomputation, adjoint)")
         roofline["traffic_over_algorithmic"] = round(traffic / max(algo_per_launch, 1.0), 3)
-    per_kernel = {k: {"achieved_GBps": round(v[0] / v[2] / (v[1] / 1e3) / 1e9, 1) if v[1] else None,
+    if resident:
+        roofline = resident_report(tiling, N, avg_ms, n, timed, args.steps * nt * passes)
+    per_kernel = {k: {"achieved_GBps": round(v[0] / v[2] / (v[1] / 1e3) / 1e9, 1) if v[1] and not resident else None,
                       "launches": v[2], "timed_launches": v[3], "avg_launch_ms": round(v[1], 4),
                       "est_total_ms": round(v[1] * v[2], 1)} for k, v in kern.items()}
     ms_step = wall / K * 1e3
     sim.close()
-    if copy:
+    if copy and not resident:
         roofline["copy_GBps"] = round(copy, 1)
         roofline["copy_probe"] = "torch elementwise multiply, 1 GiB in, 1 GiB out, this GPU"
         roofline["frac_of_copy"] = round(achieved / copy, 4)
@@ -512,7 +526,7 @@ def main():
 
     value = 2.0 * cells * nt * shots_timed / wall / 1e9
     shots_per_s = shots_timed / wall
-    hbm_frac = model_bytes * nt * shots_timed / wall / HBM_PEAK
+    hbm_frac = None if resident else round(model_bytes * nt * shots_timed / wall / HBM_PEAK, 4)
 
     plain = None
     if not args.no_plain:
@@ -557,7 +571,7 @@ def main():
             cpu = {"skipped": f"past the {args.deadline:.0f} s deadline"}
 
     # the stencil's own access shape, on the batch's array size (after the contexts are closed)
-    if not args.no_probes and have_time(20.0):
+    if not args.no_probes and not resident and have_time(20.0):
         shape = shape_bandwidth(nz, (nx + 1 + 63) // 64 * 64, int(plan["batch"]))
         if shape:
             roofline["shape_GBps"] = round(shape, 1)
@@ -588,7 +602,7 @@ def main():
                    "ckpt_kept": plan["ckpt_kept"], "recompute": plan["recompute"], "snap_dt": sdt, "tile_rows": tz,
                    "parallelism": "single GPU, shots batched per launch"},
         "shots_per_s": round(shots_per_s, 3),
-        "hbm_frac": round(hbm_frac, 4),
+        "hbm_frac": hbm_frac,
         "roofline": roofline,
         "kernels": per_kernel,
         "timed_run": (f"eager launches; HIP events on every {args.event_stride}-th launch of each stencil kernel "

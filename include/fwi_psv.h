@@ -229,7 +229,9 @@ enum fwi_kernel_id {
     FWI_K_RECEIVER = 4,   /* urec2 */
     FWI_K_STORE = 5,      /* gard_fwd_storage2 / checkpoint copies */
     FWI_K_OTHER = 6,
-    FWI_K_STEP = 7,       /* one-pass time step: stress, top free surface and velocity (kernel variant 4) */
+    FWI_K_STEP = 7,       /* one-pass time step: stress, top free surface and velocity (variants 4, 7 to 9);
+                             or a range of time steps of the resident propagation, one launch each
+                             (fwi_resident_tiling), whose seismogram sums count as FWI_K_RECEIVER */
     FWI_K_GRAPH = 8,      /* a replayed hipGraph of several whole time steps (use_graph) */
     FWI_K_COUNT = 9
 };

@@ -2,9 +2,12 @@
 what the kernels assume of it, and the forms that the GPU tests name take the kernels they name.
 """
 import random
+import sys
 
 import numpy as np
 import pytest
+
+from conftest import ROOT
 
 # nz, nx, order, shots, free surface, CPML cells: cells per thread on 256 compute units, and more of
 # the tiling where a test is there for it
@@ -118,3 +121,16 @@ def test_plan_tiling_refuses_bad_arguments():
         assert e.value.status == -1
     with pytest.raises(_lib.FwiError):
         psv.plan_tiling(40, 40, 8, 1, cus=0)
+
+
+def test_bench_reports_resident_launches_per_time_step():
+    """bench.py makes no HBM bandwidth of launches that keep their fields on the chip: it names the
+    resident kernel and gives the time of a time step."""
+    sys.path.insert(0, str(ROOT))
+    import bench
+    t = dict(cells=0, shots=2)
+    r = bench.resident_report(t, 4, 6.8, 10, 5, 20000)
+    assert r["instantiation"] == "k_resident1<4, *>" and r["us_per_time_step"] == 3.4 and r["tiling"] is t
+    assert r["achieved"] is r["frac"] is r["peak"] is None
+    for cells, name in ((1, "k_resident<float, 6, 1, 32, *>"), (4, "k_resident<float, 6, 4, 64, *>")):
+        assert bench.resident_report(dict(t, cells=cells), 6, 1.0, 1, 1, 100)["instantiation"] == name
