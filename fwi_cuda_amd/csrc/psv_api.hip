@@ -143,10 +143,13 @@ struct fwi_ctx {
     // plain form: full-grid derivative scratch and CPML memory (one shot)
     bool plain = false;
     PlainBufs pb{};
-    bool tuned = false;
-    int var = 2;   // stencil kernel variant (autotuned); 4 = one-pass step
+    int var = 2;   // stencil kernel variant of the running pass (autotuned); 4 = one-pass step
     int order = 0; // stencil work order (autotuned)
     int depth = 1; // rows the one-pass step loads ahead (autotuned)
+    struct Choice {
+        bool tuned = false;
+        int var, tz, depth, order;
+    } choice[2];   // for batches up to Bg; for the larger ones of a forward pass
     std::string tune_log;
 
     // ---- the resident propagation (psv_resident.h): tilings per batch size
@@ -772,14 +775,21 @@ int check_finite(fwi_ctx *c, int nb) {
 }
 
 // Autotuner: kernel variant, rows per thread (TZ) and work order of the two
-// stencil kernels, timed on a gradient's batch (zeroed state, a few steps per candidate);
-// the best is kept per (grid, order, batch) for the process, and a context keeps what its
-// first pass got for all its passes, whatever their number of shots: a gradient's batches, its
-// misfit and the trials it is compared with then come from one kernel.
+// stencil kernels, timed on the batch (zeroed state, a few steps per candidate); the best is
+// kept per (grid, order, batch) for the process.  A context tunes at most twice, whatever the
+// batches its calls make: for a gradient's batch, which all smaller ones share, and where a
+// forward pass takes more shots at once, for that batch by forward steps alone (snapshots and
+// sums hold a gradient's batch).  Which kernel is best changes with the batch: at 1001 x 2001 a
+// forward pass of 8 shots takes 92 ms with what forward steps of 8 shots choose (variant 13)
+// and 108 with what a gradient's batch of 4 does (variant 12).  The second choice keeps the
+// first's kind: the two-kernel variants and the resident kernels give the same seismograms bit
+// for bit, the one-pass ones do among themselves (below z strips), so that the misfit of a
+// gradient and of its trial steps compare exactly.
 struct TuneKey {
     int nz, nx, N, B;
+    bool fwd;
     bool operator<(const TuneKey &o) const {
-        return std::tie(nz, nx, N, B) < std::tie(o.nz, o.nx, o.N, o.B);
+        return std::tie(nz, nx, N, B, fwd) < std::tie(o.nz, o.nx, o.N, o.B, o.fwd);
     }
 };
 struct TuneVal {
@@ -788,24 +798,42 @@ struct TuneVal {
 std::map<TuneKey, TuneVal> g_tuned;
 std::mutex g_tune_mu;
 
-void take(fwi_ctx *c, const TuneVal &v) {
+// the running pass's kernel: choice i
+void use(fwi_ctx *c, int i) {
+    const auto &v = c->choice[i];
     c->var = v.var;
     c->tz = v.tz;
     c->depth = v.depth;
     c->order = v.order;
-    c->tuned = true;
 }
 
-int autotune(fwi_ctx *c) {
-    if (c->plain || c->tuned) return FWI_OK;
-    const int nb = c->Bg;   // what the snapshots and sums hold
-    const TuneKey key{c->g.nz, c->g.nx, c->N, nb};
+void take(fwi_ctx *c, int i, const TuneVal &v) {
+    c->choice[i] = {true, v.var, v.tz, v.depth, v.order};
+    use(c, i);
+}
+
+// the kernel of a pass over n shots at once, tuned if need be
+int autotune(fwi_ctx *c, int n) {
+    if (c->plain) return FWI_OK;
+    const int ci = n > c->Bg;
+    const bool fwd = ci == 1;
+    if (c->choice[ci].tuned) {
+        use(c, ci);
+        return FWI_OK;
+    }
+    const int nb = fwd ? c->B : c->Bg;
+    const auto &other = c->choice[1 - ci];
+    // the other batch's kind of kernel, where it has one
+    const bool two_kernel = c->B > c->Bg && (other.tuned ? !one_pass(other.var) : resident(c, fwd ? c->Bg : c->B));
+    const bool single = c->B > c->Bg && other.tuned && one_pass(other.var);
+    auto of_kind = [&](int var) { return one_pass(var) ? !two_kernel : !single; };
+    const TuneKey key{c->g.nz, c->g.nx, c->N, nb, fwd};
     const int fv = c->o.kernel_variant;   // 0 = any
     const bool order_forced = c->o.work_order >= 1 && c->o.work_order <= 4;
     // candidates (variant, rows per segment, prefetch depth); the one-pass step only where it applies
     std::vector<TuneVal> cand;
     for (int var = 1; var <= 13; ++var) {
-        if ((fv && var != fv) || (one_pass(var) && !c->fusable) || (var >= 5 && !c->ztab_ok)) continue;
+        if ((fv && var != fv) || !of_kind(var) || (one_pass(var) && !c->fusable) || (var >= 5 && !c->ztab_ok)) continue;
         if (var == 9) {   // balanced: one or two waves of resident blocks
             for (int m : {1, 2})
                 if (c->o.tile_tz <= 0 || c->o.tile_tz == m) cand.push_back({9, m, 1, 2});
@@ -837,16 +865,16 @@ int autotune(fwi_ctx *c) {
                                    "variant 4's conditions and variant 6's z CPML strips)"
                                  : "");
     if (cand.size() == 1 && order_forced) {   // nothing left to choose
-        take(c, {cand[0].var, cand[0].tz, cand[0].depth, c->o.work_order - 1});
+        take(c, ci, {cand[0].var, cand[0].tz, cand[0].depth, c->o.work_order - 1});
         return FWI_OK;
     }
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
         auto it = g_tuned.find(key);
-        if (it != g_tuned.end() && (!fv || fv == it->second.var) && (!one_pass(it->second.var) || c->fusable) &&
+        if (it != g_tuned.end() && (!fv || fv == it->second.var) && of_kind(it->second.var) && (!one_pass(it->second.var) || c->fusable) &&
             (!order_forced || c->o.work_order - 1 == it->second.order) &&
             (c->o.tile_tz <= 0 || c->o.tile_tz == it->second.tz)) {
-            take(c, it->second);
+            take(c, ci, it->second);
             return FWI_OK;
         }
     }
@@ -879,8 +907,8 @@ int autotune(fwi_ctx *c) {
     ap.displ = 1;
     std::vector<KArgs *> mix;
     for (int k = 0; k < kmix; ++k) mix.push_back(&a);
-    for (int k = 0; k < kmix; ++k) mix.push_back(k ? &ar : &as);
-    for (int k = 0; k < kmix; ++k) mix.push_back(k ? &ap : &ag);
+    for (int k = 0; k < kmix && !fwd; ++k) mix.push_back(k ? &ar : &as);
+    for (int k = 0; k < kmix && !fwd; ++k) mix.push_back(k ? &ap : &ag);
     auto run = [&](const TuneVal &v) {
         for (KArgs *x : mix) {
             x->order = a.order;
@@ -918,7 +946,7 @@ int autotune(fwi_ctx *c) {
     }
     hipEventDestroy(e0);
     hipEventDestroy(e1);
-    take(c, bv);
+    take(c, ci, bv);
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tuned[key] = bv;
     return FWI_OK;
@@ -927,7 +955,7 @@ int autotune(fwi_ctx *c) {
 // Forward pass (kernel_PSV with grad = false) for shots [s0, s0 + nb).
 int run_forward(fwi_ctx *c, int s0, int nb, bool store, bool record, bool energy) {
     const bool res = resident(c, nb);
-    if (!res) RETIF(autotune(c));
+    if (!res) RETIF(autotune(c, nb));
     const Wave w = main_wave(c);
     RETIF(zero_state(c, nb, w, true, !res));
     if (record) HIPCHK(hipMemsetAsync(c->acc, 0, sizeof(double) * 2 * c->nrec_tot, c->st));
@@ -2892,7 +2920,7 @@ int32_t fwi_tuning(const fwi_ctx *c, int32_t *tile_tz, char *log, int32_t log_le
     if (log && log_len > 0) {
         char head[64];
         std::snprintf(head, sizeof head, "chosen o%d/v%d/tz%d/d%d; ", c->order, c->var, c->tz, c->depth);
-        const std::string s = (c->tuned ? std::string(head) : std::string()) + c->tune_log;
+        const std::string s = (c->choice[0].tuned || c->choice[1].tuned ? std::string(head) : std::string()) + c->tune_log;
         std::strncpy(log, s.c_str(), (size_t)log_len - 1);
         log[log_len - 1] = 0;
     }

@@ -95,6 +95,39 @@ def test_tuned_once_per_context(psv, O):
                 assert sim.tuning()[1] == log
 
 
+@pytest.mark.parametrize("first", ["forward", "gradient"])
+def test_two_batches_tune_once_each(psv, O, first):
+    """Where a forward pass takes more shots at once than a gradient, each of the two batches is
+    tuned once, whichever comes first, for kernels whose misfits compare exactly."""
+    c = cases.small_case(O, nz=500, nx=700, nt=40, nshot=8, snap_dt=1)
+    obs = _obs(c)
+    with psv.Simulation(c, storage=psv._lib.STORE_FULL, kernel_variant=5) as sim:
+        budget = int(0.6 * sim.plan()["device_bytes"])
+    with psv.Simulation(c, mem_budget=budget, work_order=1) as sim:   # a pinned order: launch by launch
+        p = sim.plan()
+        assert p["gradient_batch"] < p["batch"] and sim.resident_tiling()["shots"] == 0
+        sim.set_observed(*obs)
+        heads = {}
+        for k in range(2):
+            for what in (first, *{"forward", "gradient"} - {first}):
+                m = sim.gradient() if what == "gradient" else sim.misfit()
+                if what == "gradient":
+                    total = sum(m.tolist())
+                else:
+                    misfit = m
+                head, *log = sim.tuning()[1].split("; ")
+                assert heads.setdefault(what, head) == head
+            if k == 0:
+                timed = log
+        assert total == misfit
+        for call in (lambda: sim.forward(0, 3), lambda: sim.gradient(0, 2), lambda: sim.forward()):
+            call()
+            assert sim.tuning()[1].split("; ")[1:] == timed
+        one_pass = [int(h.split("/v")[1].split("/")[0]) in (4, 7, 8, 9) for h in heads.values()]
+        assert one_pass[0] == one_pass[1]
+        print(first, heads, len(timed), flush=True)
+
+
 def test_gradient_batch_smaller_than_forward_batch(psv, O):
     """With storage and batch left open and memory for part of the snapshots, a gradient runs in
     smaller batches than a forward pass: same bits as contexts whose one batch holds all shots or
