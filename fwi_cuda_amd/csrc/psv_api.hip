@@ -1462,8 +1462,8 @@ constexpr int kMaxUnits = 2048;   // the schedule's dynamic programme is O(units
 // of all shots costs each pass's launches (16 us a batch) and cells (forward and adjoint 33
 // us per million, a recomputed step 12 more), and a smaller batch recomputes less or
 // nothing.  The fields still hold c->B shots, for forward passes.  Measured per gradient:
-// 1001 x 2001, 8 shots, 480 steps in 24 GB 374 ms as one checkpointed batch, 324 as two
-// full ones; 2001 x 4001, 2 shots, 240 steps in 16 GB 224 and 195.
+// 1001 x 2001, 8 shots, 480 steps in 24 GB 341 ms as one checkpointed batch, 320 as three
+// full ones; 2001 x 4001, 2 shots, 240 steps in 16 GB 214 as one and 183 as two.
 int plan_gradient_batch(fwi_ctx *c, int storage, int S, int slots, int units, size_t budget) {
     const double cells = 1e-6 * c->g.nz * c->g.nx * c->nshot;
     // recomputed share of the steps with batches of b shots, or -1 if they do not fit

@@ -8,11 +8,11 @@
 // Per half-step a block publishes its tile's edges and reads its neighbours'; nothing else
 // leaves the chip but snapshots and receiver samples.  A step is then bound by the two edge
 // exchanges (about 1.3 us each: a store to memory and a load from it, across the XCDs)
-// and, from some 1000 cells per CU on, by the cells a thread computes.  Measured per forward
-// step, launch-by-launch and resident: 72 x 96, 3 shots 16.4 -> 4.0 us; 201 x 401 17.9 -> 3.8;
-// the FP64 propagation at 201 x 401 beside the FP32 one 37 -> 8.9; per gradient step
-// (forward and adjoint) 201 x 401 37.5 -> 8.1, 246 x 335 order 4, 3 shots 36.6 -> 11.8, 301 x
-// 601, 8 shots 90 -> 50 (two launches of four shots).
+// and, from some 1000 cells per CU on, by the cells a thread computes.  Measured per time step
+// of a call, launch by launch and resident: forward 72 x 96, 3 shots 16.4 -> 3.1 us, 201 x 401
+// 17.7 -> 3.4 (both by k_resident1 below); the FP64 propagation at 201 x 401 beside the FP32 one
+// 37 -> 8.9; a gradient (forward and adjoint) 201 x 401 37.5 -> 7.0, 246 x 335 order 4, 3 shots
+// 36.6 -> 11.1, 301 x 601, 8 shots 90 -> 50.5 (two launches of four shots).
 //
 // Exchange.  An edge value travels as one 64-bit word {value, tag} (two for FP64, each
 // half with its tag), stored and loaded with relaxed agent-scope atomics, so that one
@@ -722,7 +722,7 @@ __global__ __launch_bounds__(1024) void k_resident(const ResArgs<T> r) {
 // values as their owner, so the same bits); only velocities travel, 2N cells deep.  A step
 // then waits once instead of twice, for N more rows and columns of stress arithmetic each
 // side and more words: worth it where a CU has threads to spare (at most 32 - 2N rows and
-// columns per tile).  A tile's words are its own lines of memory, two sets taken in turn: a block
+// 31 - 2N columns per tile).  A tile's words are its own lines of memory, two sets taken in turn: a block
 // overwrites the words of step n in step n + 2, after it has seen every neighbour's words
 // of step n + 1, which they write after the barrier that follows their reads of step n.
 // The rim is loaded from arrays that its owners overwrite when they end: a block stores its
@@ -730,12 +730,12 @@ __global__ __launch_bounds__(1024) void k_resident(const ResArgs<T> r) {
 // loads.  From two steps on the exchange sees to that; a launch of one step makes the
 // exchange for that alone (k_resident waits for stress words in every step, and the exact
 // adjoint's sweep loads own cells only).
-// Measured per forward step against two exchanges: 72 x 96, 3 shots 4.1 -> 3.2 us, 201 x 401
-// 4.1 -> 3.7; forward and adjoint step 201 x 401 8.7 -> 7.5.  The FP64 propagation's words
-// are twice as many: 10.1 -> 11.1, so it keeps the two exchanges.  A tile's words lie
-// together: at their cell's place in one array (lines written by several blocks) 17 x 15
-// tiles took 4.4 instead of 3.9; rows of 32 lanes: packed to the tile's width they take
-// fewer wavefronts but 4.0 instead of 3.7.
+// Measured per time step of a call, two exchanges and one: 72 x 96, 3 shots 4.2 -> 3.1 us, 201 x
+// 401 3.8 -> 3.4; forward and adjoint 201 x 401 8.1 -> 7.0.  The FP64 propagation's words are
+// twice as many: with one exchange its step took a tenth longer, so it keeps two.  A tile's
+// words lie together: at their cell's place in one array (lines written by several blocks) a
+// step of 17 x 15 tiles took an eighth longer; rows of 32 lanes: packed to the tile's width
+// they take fewer wavefronts, and a step 8 % longer.
 template <int N, bool ADJ>
 __global__ __launch_bounds__(1024) void k_resident1(const ResArgs<float> r) {
     extern __shared__ char smem[];

@@ -49,16 +49,18 @@ int strip_lines(const std::vector<int> &map, int N, int T) {
 }  // namespace
 
 // The tiling that takes the least time for nb shots on cus compute units with lds bytes each,
-// by measured step times in us: a base (the barriers and latencies of the chain of a thread's
-// cells, and the two edge exchanges) and a slope per lane-cell of the block.  One cell per
+// by a model of step times in us: a base (the barriers and latencies of the chain of a thread's
+// cells, and the two edge exchanges) and a slope per lane-cell of the block, fitted to sweeps of
+// tiles (of use to compare them, not for a call's time).  Measured there with one cell per
 // thread: 3.8 at 300 cells, 4.4 at 740; two: 5.6 at 450, 6.5 at 1600; four: 10.8 at 3300;
 // eight (its registers spill): 25 at 4600.  FP64 and the exact adjoint's sweep cost what
 // their registers and words do; that sweep with four cells per thread spills its FP64 sums
-// (301 x 601, 4 shots: 31 us a step against 2 x 10 for two launches of two cells per
-// thread).  Every tile holds at least N rows and columns (its halo comes from direct
-// neighbours only; the one-exchange kernel, 0 cells per thread, has none such).  FP32 steps that the batched kernels run as fast, at 16 us of launches
-// and 14.4 us per million cells, are left to them: 600 x 1100, 8 shots take 78 us there and
-// 82 here, 800 x 1400, 1 shot 35 and 26.
+// (301 x 601, 4 shots: 31 us a step against 2 x 11.5 for two launches of two cells per
+// thread).  Every tile holds at least N rows and columns, as its halo comes from direct
+// neighbours only (the one-exchange kernel, 0 cells per thread, reads any tile's words).  FP32
+// steps that the batched kernels run as fast, at 16 us of launches and 14.4 us per million
+// cells, are left to them: 600 x 1100, 8 shots take 78 us there and 82 here, 800 x 1400, 1
+// shot 35 and 26.
 bool plan_resident(int nz, int nx, int N, int nb, ResUse use, int cus, size_t lds, const std::vector<int> &zmap,
                    const std::vector<int> &xmap, ResPlan *out) {
     const int elt = use == kUseFp64 ? 8 : 4, fields = use == kUseExact ? 4 : 5;
@@ -75,8 +77,8 @@ bool plan_resident(int nz, int nx, int N, int nb, ResUse use, int cus, size_t ld
             const int cols = strip_lines(xmap, N, TX);
             for (int ntz = 1; ntz <= std::min(tiles / ntx, iz); ++ntz) {
                 // one exchange per step (a single tile has none: one cell per thread); tiles that
-                // fill the 32 lanes measured 5 % slower than the next narrower ones (201 x 401:
-                // 24 x 13 cells 3.9 us, 22 x 14 3.7, 16 x 20 3.7)
+                // fill the 32 lanes measured 5 % slower than narrower ones (201 x 401: 24 x 13
+                // cells against 22 x 14 and 16 x 20, which take the same time)
                 if (use != kUseExact && use != kUseFp64 && TX + 2 * N < 32 && ntx * ntz > 1) {
                     const int TZ = (iz + ntz - 1) / ntz;
                     const int thr = (32 * (TZ + 2 * N) + 63) / 64 * 64;

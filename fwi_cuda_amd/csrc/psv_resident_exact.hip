@@ -7,9 +7,9 @@
 // carries and the FP64 media gradient stay in registers (carries of tall threads in LDS),
 // and LDS holds the four derivative adjoints of one half-step, whose z and x gathers need
 // the neighbours' edge rows and columns.  The step's history is read ahead of the waits.
-// Bound by the exchanges and barriers: 6.3 us a step at 201 x 401, 10 per launch of two
-// shots at 301 x 601.  A call (its forward passes included): 201 x 401, 800 steps 63.5 ->
-// 11.9 ms; 301 x 601, 4 shots, 400 steps 65.6 -> 19.6 ms, both with the workspace kept.
+// Bound by the exchanges and barriers: 6.0 us a step at 201 x 401; by issue beside them: 11.5
+// per launch of two shots at 301 x 601.  A call with the forward pass before it: 201 x 401, 800
+// steps 63.4 -> 11.4 ms; 301 x 601, 4 shots, 400 steps 66.4 -> 19.4 ms, with the workspace kept.
 // Same operations in the same order and with the same fused products as psv_exact.hip's
 // kernels, for no free surface or the
 // top one at row N (no image rows) and points inside the interior; other set-ups keep
