@@ -431,3 +431,44 @@ def test_contexts_on_several_threads(psv, O):
         for r in runs:
             for a, b in zip(r, w):
                 np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("stf_type", [0, 1])
+@pytest.mark.parametrize("form", [(90, 140, 8, 3), (246, 335, 8, 2), (246, 335, 4, 3), (321, 611, 4, 5)],
+                         ids=lambda f: f"{f[0]}x{f[1]}-o{f[2]}x{f[3]}")
+def test_points_of_any_number_and_place(psv, O, form, stf_type):
+    """Shots with several sources and receivers of their own, some in one cell, some on the first and
+    last cells of the interior and of tiles: bit for bit variant 5, units of one step included."""
+    nz, nx, order, ns = form
+    N = order // 2
+    c = cases.small_case(O, nz=nz, nx=nx, nt=61, fdorder=order, nshot=ns, snap_dt=1)
+    rng = np.random.default_rng(nz + order + stf_type)
+    with psv.Simulation(c) as sim:
+        t = sim.resident_tiling()
+    edge_z = [N, nz - N - 1, min(N + t["rows"], nz - N - 1), min(N + t["rows"] - 1, nz - N - 1)]
+    edge_x = [N, nx - N - 1, min(N + t["cols"], nx - N - 1), min(N + t["cols"] - 1, nx - N - 1)]
+    z, x, fire, zr, xr, off = [], [], [], [], [], [0]
+    for s in range(ns):
+        z += [N + 3 + s, N + 3 + s, *edge_z[:3], int(rng.integers(N, nz - N))]
+        x += [nx // 2, nx // 2, *edge_x[1:], int(rng.integers(N, nx - N))]
+        fire += [s] * 6
+        zr += [N + 3 + s, N + 3 + s, *edge_z, N + 1][s:]   # shot s has 7 - s receivers
+        xr += [nx // 2, nx // 2, *edge_x, nx // 2 + 2][s:]
+        off.append(len(zr))
+    w = rng.uniform(-1.0, 1.0, (2, len(z), 1)) * c["stf_z"][:1]
+    c.update(z_src=np.array(z, np.int32), x_src=np.array(x, np.int32), shot_to_fire=np.array(fire, np.int32),
+             stf_z=np.ascontiguousarray(w[0]), stf_x=np.ascontiguousarray(w[1]), stf_type=stf_type,
+             z_rec=np.array(zr, np.int32), x_rec=np.array(xr, np.int32), rec_off=np.array(off, np.int32))
+    obs = [1e-13 * rng.standard_normal((off[-1], 61)) for _ in range(2)]
+    out = []
+    for kw in (dict(kernel_variant=5), {}, dict(storage=psv._lib.STORE_CHECKPOINT, ckpt_interval=12, ckpt_keep=1)):
+        with psv.Simulation(c, **kw) as sim:
+            assert (sim.resident_tiling()["shots"] > 0) == ("kernel_variant" not in kw)
+            seis = sim.forward()
+            sim.set_observed(*obs)
+            out.append((*seis, sim.gradient(), *sim.get_gradient(), *sim.misfit_gradient(*obs),
+                        *sim.misfit_gradient_exact(*obs)))
+    for o in out[1:]:
+        for i, (a, b) in enumerate(zip(o, out[0])):
+            assert np.abs(b).max() > 0
+            np.testing.assert_array_equal(a, b, err_msg=f"output {i}")
