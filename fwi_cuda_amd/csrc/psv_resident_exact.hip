@@ -10,8 +10,9 @@
 // Bound by the exchanges and barriers: 6.0 us a step at 201 x 401; by issue beside them: 11.5
 // per launch of two shots at 301 x 601.  A call with the forward pass before it: 201 x 401, 800
 // steps 63.4 -> 11.4 ms; 301 x 601, 4 shots, 400 steps 66.4 -> 19.4 ms, with the workspace kept.
-// Same operations in the same order and with the same fused products as psv_exact.hip's
-// kernels, for no free surface or the
+// Same operations in the same order as psv_exact.hip's kernels, with their fused products but
+// for one (d3; over 8 seeds of 201 x 401 its form here leaves lam, mu errors of 1.61, 2.01e-6
+// against 64 bits, theirs 1.66, 2.18e-6), for no free surface or the
 // top one at row N (no image rows) and points inside the interior; other set-ups keep
 // those kernels.
 #include "psv_resident.h"
@@ -264,7 +265,7 @@ __global__ __launch_bounds__(1024) void k_resident_exact(const ResExact r) {
                 G[2][k] = fmadd((double)dt * zx, (double)e_zx, G[2][k]);
                 const float lu = fmadd(2.f, u, l);
                 float d0 = dt * fmadd(l, xx, lu * zz);
-                float d3 = fmadd(dt, fmadd(l, zz, lu * xx), s3);
+                float d3 = fmadd(dt, fmadd(lu, xx, l * zz), s3);   // the larger product fused: as one cell per thread had it
                 float d1 = dt * muzx[k] * zx, d2 = d1;
                 if (zin >> k & 1) {
                     const float *p = zprof + (zv + k) * 6;
