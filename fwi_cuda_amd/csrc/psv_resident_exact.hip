@@ -11,10 +11,9 @@
 // per launch of two shots at 301 x 601.  A call with the forward pass before it: 201 x 401, 800
 // steps 63.4 -> 11.4 ms; 301 x 601, 4 shots, 400 steps 66.4 -> 19.4 ms, with the workspace kept.
 // Same operations in the same order as psv_exact.hip's kernels, with their fused products but
-// for one (d3; over 8 seeds of 201 x 401 its form here leaves lam, mu errors of 1.61, 2.01e-6
-// against 64 bits, theirs 1.66, 2.18e-6), for no free surface or the
-// top one at row N (no image rows) and points inside the interior; other set-ups keep
-// those kernels.
+// for one (d3; over eight models of 201 x 401 its form here leaves lam, mu errors of 1.61,
+// 2.01e-6 against 64 bits, theirs 1.66, 2.18e-6), for no free surface or the top one at row N
+// (no image rows) and points inside the interior; other set-ups keep those kernels.
 #include "psv_resident.h"
 
 namespace psv {
